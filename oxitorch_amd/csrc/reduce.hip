@@ -3,18 +3,22 @@
 // (crates/oxi-tensor/src/ops.rs:246-285) and Tensor::reduce
 // (crates/oxi-tensor/src/lib.rs:519-576).
 //
-// Two kernels:
-//   strip-contiguous (reduced dim has stride 1): one wave64 per strip, lanes
-//     stride the strip, shuffle-tree combine;
-//   strided (any other stride): one thread per output element walking its
-//     strip in order; for sum/mean/norm this is the reference's own
-//     sequential f32 fold, so the result is bit-identical to it. Adjacent
-//     threads own adjacent output elements, so a column reduction of a
-//     row-major tensor reads coalesced rows.
+// Kernels:
+//   strip-contiguous (reduced dim has stride 1): a wave, or for long strips a
+//     block, per strip; lanes read the strip as float4s at any float
+//     alignment, four in flight, and the group combines in a fixed tree. Few
+//     long strips are cut into parts over the chip, combined by a second
+//     launch;
+//   strided (any other stride): for sum/mean/norm every output is the
+//     reference's own sequential f32 fold over its strip, so the result is
+//     bit-identical to it. Many outputs: a thread walks the strip of one or
+//     four adjacent outputs. Few outputs: a block stages the strips of 16
+//     adjacent outputs through LDS and one lane per output folds them.
 // max/min fold with fmaxf/fminf (NaN ignored, as f32::max/min); argmax/argmin
 // keep the first strict winner starting from index 0, so a NaN at index 0
 // sticks and later NaNs are ignored. Indices are written as floats.
 #include <algorithm>
+#include <type_traits>
 
 #include "internal.h"
 #include "rowtile.h"
@@ -24,6 +28,31 @@ namespace {
 
 constexpr int BS = 256;
 constexpr int MAXD = OXI_MAX_DIMS;
+
+// Where the launch shapes change, with times on MI355X (before: one wave per
+// contiguous strip reading single floats, one thread per output or four).
+// Contiguous strips of up to WAVE_MAX_LEN floats take a wave each (mean over
+// (16384, 768) 16.3 -> 8.9 us), longer ones a block of 256 threads, or 1024
+// while there are under two strips per CU: argmax over (4096, 50257) 438 ->
+// 128 us, sum over (64, 16384) 31.6 -> 4.3 us.
+constexpr int64_t WAVE_MAX_LEN = 2048;
+// From SPLIT_MIN_LEN on, and with fewer strips than CUs, the strips are cut
+// into parts of a multiple of SPLIT_MIN_PART floats (four float4s a thread),
+// about SPLIT_BLOCKS_PER_CU a CU in all: the norm of 12.6M values 46000 ->
+// 12.9 us (3.9 TB/s), 1M values 1560 -> 7.1 us. The second launch costs about
+// 3 us, what one block takes for 30000 floats more.
+constexpr int64_t SPLIT_MIN_LEN = 65536;
+constexpr int64_t SPLIT_BLOCKS_PER_CU = 4;
+constexpr int64_t SPLIT_MIN_PART = 4096;
+// Strided strips of COLS_MIN_LEN positions or more, of up to COLS_MAX_OUT
+// outputs, go through LDS: the column sums of (16384, 768) 758 -> 59 us, of
+// (1024, 16384) 68 -> 25 us, of (4096, 8000) 298 -> 42 us, the maxima of
+// (16384, 768) 760 -> 38 us. With more outputs a thread per output fills the
+// chip: (512, 65536) 42 us there against 57 us through LDS. Two and four
+// stages of loads in flight instead of one: 61-90 us at (16384, 768), the
+// staging then holding up the fold.
+constexpr int64_t COLS_MIN_LEN = 64;
+constexpr int64_t COLS_MAX_OUT = 16384;
 
 struct RPlan {
   int nd;              // dims other than the reduced one
@@ -71,6 +100,11 @@ struct Acc {
   }
 };
 
+// One thread per output. The loads of STRIDED_U positions issue together and
+// are folded in order: the column sums of (512, 50001) 128 -> 19 us (8: 27 us).
+constexpr int STRIDED_U = 16;
+constexpr int VEC_U = 8;  // the same for four outputs a thread (16: as fast)
+
 template <int K>
 __global__ __launch_bounds__(BS) void reduce_strided_k(const float* __restrict__ x, RPlan p, int64_t nout,
                                                        float* __restrict__ out) {
@@ -78,9 +112,178 @@ __global__ __launch_bounds__(BS) void reduce_strided_k(const float* __restrict__
     const float* s = x + base_of(p, e);
     Acc<K> a;
     a.init(p.len ? s[0] : 0.f);
-    for (int64_t k = 0; k < p.len; ++k) a.add(s[k * p.rst], k);
+    int64_t k = 0;
+    for (; k + STRIDED_U <= p.len; k += STRIDED_U) {
+      float v[STRIDED_U];
+#pragma unroll
+      for (int u = 0; u < STRIDED_U; ++u) v[u] = s[(k + u) * p.rst];
+#pragma unroll
+      for (int u = 0; u < STRIDED_U; ++u) a.add(v[u], k + u);
+    }
+    for (; k < p.len; ++k) a.add(s[k * p.rst], k);
     out[e] = a.result(p.len);
   }
+}
+
+constexpr bool is_arg(int k) { return k == OXI_REDUCE_ARGMAX || k == OXI_REDUCE_ARGMIN; }
+// kinds whose result depends on the order of the fold
+constexpr bool is_fold(int k) { return k == OXI_REDUCE_SUM || k == OXI_REDUCE_MEAN || k == OXI_REDUCE_NORM; }
+
+// The state of one lane or group over part of a strip. For
+// argmax/argmin it is the first winner among non-NaN values; a NaN at
+// position 0 of the strip forces index 0, matching the sequential scan.
+template <int K>
+struct Part {
+  float v;    // arg*: the winner, NaN while there is none
+  int64_t i;  // arg*: its position
+  static __device__ __forceinline__ Part none() {
+    if constexpr (K == OXI_REDUCE_MAX) return {-__builtin_huge_valf(), 0};
+    else if constexpr (K == OXI_REDUCE_MIN) return {__builtin_huge_valf(), 0};
+    else if constexpr (is_arg(K)) return {__builtin_nanf(""), 0};
+    else return {0.f, 0};
+  }
+  __device__ __forceinline__ void add(float a, int64_t k) {
+    if constexpr (K == OXI_REDUCE_SUM || K == OXI_REDUCE_MEAN) v += a;
+    else if constexpr (K == OXI_REDUCE_NORM) v += a * a;
+    else if constexpr (K == OXI_REDUCE_MAX) v = fmaxf(v, a);
+    else if constexpr (K == OXI_REDUCE_MIN) v = fminf(v, a);
+    else {
+      // not (a <= v): a strict winner, or the first (v is NaN)
+      const bool better = !((K == OXI_REDUCE_ARGMAX) ? (a <= v) : (a >= v)) & (a == a);
+      v = better ? a : v;
+      i = better ? k : i;
+    }
+  }
+  // o may hold positions before or after this one's: a tie goes to the smaller index
+  __device__ __forceinline__ void merge(const Part& o) {
+    if constexpr (is_fold(K)) v += o.v;
+    else if constexpr (K == OXI_REDUCE_MAX) v = fmaxf(v, o.v);
+    else if constexpr (K == OXI_REDUCE_MIN) v = fminf(v, o.v);
+    else {
+      const bool better = !((K == OXI_REDUCE_ARGMAX) ? (o.v <= v) : (o.v >= v)) & (o.v == o.v);
+      if (better || (o.v == v && o.i < i)) *this = o;
+    }
+  }
+};
+
+// The state of the lane whose number differs by the mask m.
+template <int K>
+__device__ __forceinline__ Part<K> part_xor(const Part<K>& a, int m) {
+  Part<K> o = Part<K>::none();
+  o.v = __shfl_xor(a.v, m, 64);
+  if constexpr (is_arg(K)) o.i = __shfl_xor(a.i, m, 64);
+  return o;
+}
+
+template <int K>
+__device__ __forceinline__ float strip_result(const float* s, const Part<K>& a, int64_t len) {
+  if constexpr (K == OXI_REDUCE_MEAN) return a.v / (float)len;
+  else if constexpr (K == OXI_REDUCE_NORM) return sqrtf(a.v);
+  else if constexpr (is_arg(K)) return (s[0] != s[0]) ? 0.f : (float)a.i;
+  else return a.v;
+}
+
+// Few outputs over long strips: a block owns COLS_C outputs adjacent in
+// memory. Its loading threads take COLS_R positions of them at a time
+// (coalesced rows of 64 bytes) and store them transposed in LDS, where the
+// lanes of one more wave, one per output, fold their strips in order; the next
+// positions' loads are in flight meanwhile, and two LDS stages alternate, so
+// there is one barrier a stage. What bounds it is that fold, a chain of
+// dependent adds of 8 cycles each, which the reference's order fixes (55 us
+// for 16384 positions, of the 59 us the 768 columns of such a strip take); max, min and arg* take
+// four lanes per output, each a quarter of every stage. VEC: rows of float4s
+// (columns a multiple of 4, aligned); else single floats.
+constexpr int COLS_LT = 512;   // loading threads
+constexpr int COLS_NT = COLS_LT + 64;
+constexpr int COLS_C = 16;     // outputs per block
+constexpr int COLS_R = 512;    // positions a stage
+constexpr int COLS_LD = COLS_R + 4;  // floats between outputs in LDS: 16 lanes reading float4s touch 64 distinct banks
+constexpr int COLS_F = 32;     // positions a lane has read from LDS ahead of its fold
+
+template <int K, bool VEC>
+__global__ __launch_bounds__(COLS_NT) void reduce_cols_k(const float* __restrict__ x, RPlan p, int64_t inner,
+                                                         int64_t groups, float* __restrict__ out) {
+  constexpr int W = VEC ? 4 : 1;               // floats per load
+  constexpr int TPP = COLS_C / W;              // threads per position
+  constexpr int PPP = COLS_LT / TPP;           // positions a pass of the block
+  constexpr int U = COLS_R / PPP;              // passes a stage
+  using V = typename std::conditional<VEC, f4, float>::type;
+  __shared__ __align__(16) float tile[2][COLS_C * COLS_LD];
+  const int64_t o = blockIdx.x / groups;       // row of outputs
+  const int64_t c0 = (blockIdx.x % groups) * COLS_C;
+  const int nc = (int)min<int64_t>(COLS_C, inner - c0);  // a multiple of W
+  const float* s = x + base_of(p, o * inner + c0);
+  const int64_t len = p.len, rst = p.rst;
+  if (threadIdx.x < COLS_LT) {
+    const int q = threadIdx.x % TPP, r = threadIdx.x / TPP;
+    const float* sp = s + min(q * W, nc - W);  // columns past the last output re-read it
+    V v[U];
+    auto load = [&](int64_t k0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t k = min<int64_t>(k0 + u * PPP + r, len - 1);  // positions past the strip re-read its last
+        v[u] = *reinterpret_cast<const V*>(sp + k * rst);  // plain: two blocks share a 128-byte line
+      }
+    };
+    load(0);
+    int b = 0;
+    for (int64_t k0 = 0; k0 < len; k0 += COLS_R, b ^= 1) {
+      float* t = tile[b] + q * W * COLS_LD + r;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if constexpr (VEC) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) t[j * COLS_LD + u * PPP] = v[u][j];
+        } else {
+          t[u * PPP] = v[u];
+        }
+      }
+      if (k0 + COLS_R < len) load(k0 + COLS_R);
+      // this stage is written, and the fold of the one before it is done:
+      // the next pass may overwrite that one
+      __syncthreads();
+    }
+    return;
+  }
+  // SUB lanes share an output, lane `sub` folding positions [lo, lo + COLS_R / SUB) of each stage
+  constexpr int SUB = is_fold(K) ? 1 : 64 / COLS_C;
+  const int lane = threadIdx.x & (COLS_C - 1);
+  const int lo = SUB == 1 ? 0 : (int)((threadIdx.x & 63) / COLS_C) * (COLS_R / SUB);
+  Part<K> a = Part<K>::none();
+  int b = 0;
+  for (int64_t k0 = 0; k0 < len; k0 += COLS_R, b ^= 1) {
+    __syncthreads();  // the stage is written
+    const float* c = tile[b] + lane * COLS_LD + lo;
+    const int n = (int)min<int64_t>(COLS_R / SUB, len - k0 - lo);  // <= 0: none of this stage
+    f4 fa[COLS_F / 4], fb[COLS_F / 4];
+    auto fetch = [&](f4 (&f)[COLS_F / 4], int at) {
+      const float* q = c + min(at, COLS_R / SUB - COLS_F);
+#pragma unroll
+      for (int i = 0; i < COLS_F / 4; ++i) f[i] = *reinterpret_cast<const f4*>(q + 4 * i);
+    };
+    auto fold = [&](const f4 (&f)[COLS_F / 4], int at) {
+#pragma unroll
+      for (int i = 0; i < COLS_F; ++i) a.add(f[i / 4][i % 4], k0 + lo + at + i);
+    };
+    int k = 0;
+    fetch(fa, 0);
+    // the scheduling barriers keep the next positions' reads above the adds
+    for (; k + 2 * COLS_F <= n; k += 2 * COLS_F) {
+      fetch(fb, k + COLS_F);
+      __builtin_amdgcn_sched_barrier(0);
+      fold(fa, k);
+      fetch(fa, k + 2 * COLS_F);
+      __builtin_amdgcn_sched_barrier(0);
+      fold(fb, k + COLS_F);
+    }
+    for (; k < n; ++k) a.add(c[k], k0 + lo + k);
+  }
+  if constexpr (SUB > 1) {
+#pragma unroll
+    for (int m = COLS_C; m < 64; m <<= 1) a.merge(part_xor<K>(a, m));
+  }
+  const int w = (int)threadIdx.x - COLS_LT;
+  if (w < nc) out[o * inner + c0 + w] = strip_result<K>(s + w, a, len);
 }
 
 // Four adjacent outputs per thread when they are adjacent in memory (the
@@ -95,7 +298,7 @@ __global__ __launch_bounds__(BS) void reduce_strided_vec_k(const float* __restri
     if constexpr (K == OXI_REDUCE_MAX) a = f4{-__builtin_huge_valf(), -__builtin_huge_valf(), -__builtin_huge_valf(), -__builtin_huge_valf()};
     else if constexpr (K == OXI_REDUCE_MIN) a = f4{__builtin_huge_valf(), __builtin_huge_valf(), __builtin_huge_valf(), __builtin_huge_valf()};
     else a = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
+#pragma unroll VEC_U
     for (int64_t k = 0; k < p.len; ++k) {
       const f4 v = ld_stream(reinterpret_cast<const f4*>(s + k * p.rst));
 #pragma unroll
@@ -115,85 +318,147 @@ __global__ __launch_bounds__(BS) void reduce_strided_vec_k(const float* __restri
   }
 }
 
-// Combine two partial states of a strip; (vb, ib) comes from later positions
-// only when ib > ia, so ties go to the smaller index as in the sequential scan.
-template <int K>
-__device__ __forceinline__ void combine(float& va, int64_t& ia, bool& has_a, float vb, int64_t ib, bool has_b) {
-  if constexpr (K == OXI_REDUCE_SUM || K == OXI_REDUCE_MEAN || K == OXI_REDUCE_NORM) va += vb;
-  else if constexpr (K == OXI_REDUCE_MAX) va = fmaxf(va, vb);
-  else if constexpr (K == OXI_REDUCE_MIN) va = fminf(va, vb);
-  else {
-    if (!has_b) return;
-    if (!has_a) { va = vb; ia = ib; has_a = true; return; }
-    const bool better = (K == OXI_REDUCE_ARGMAX) ? (vb > va) : (vb < va);
-    if (better || (vb == va && ib < ia)) { va = vb; ia = ib; }
+// The state over positions [k0, k1) of strip s, formed by the TPS threads of
+// a group (t = 0 .. TPS-1); thread 0 of the group returns it. Float4s at any
+// float alignment, CU_LOADS in flight per thread; each of a thread's four
+// components folds on its own and they meet in a fixed order.
+constexpr int CU_LOADS = 4;
+
+template <int K, int TPS>
+__device__ __forceinline__ Part<K> strip_part(const float* __restrict__ s, int64_t k0, int64_t k1, int t,
+                                              Part<K>* lds) {
+  constexpr int NP = is_arg(K) ? 1 : 4;  // chains per thread (arg*: one, in position order)
+  Part<K> a[NP];
+#pragma unroll
+  for (int j = 0; j < NP; ++j) a[j] = Part<K>::none();
+  const int64_t n4 = (k1 - k0) >> 2;
+  const float* p = s + k0;
+  int64_t c = t;
+  for (; c + (CU_LOADS - 1) * TPS < n4; c += CU_LOADS * TPS) {
+    f4u v[CU_LOADS];
+#pragma unroll
+    for (int u = 0; u < CU_LOADS; ++u) v[u] = ld_stream(reinterpret_cast<const f4u*>(p + 4 * (c + u * TPS)));
+#pragma unroll
+    for (int u = 0; u < CU_LOADS; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) a[j % NP].add(v[u][j], k0 + 4 * (c + u * TPS) + j);
   }
+  for (; c < n4; c += TPS) {
+    const f4u v = ld_stream(reinterpret_cast<const f4u*>(p + 4 * c));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[j % NP].add(v[j], k0 + 4 * c + j);
+  }
+  if (t < (int)((k1 - k0) & 3)) a[0].add(p[4 * n4 + t], k0 + 4 * n4 + t);
+#pragma unroll
+  for (int j = 1; j < NP; ++j) a[0].merge(a[j]);
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) a[0].merge(part_xor<K>(a[0], m));
+  if constexpr (TPS > 64) {
+    if ((t & 63) == 0) lds[t >> 6] = a[0];
+    __syncthreads();
+    if (t == 0)
+#pragma unroll
+      for (int w = 1; w < TPS / 64; ++w) a[0].merge(lds[w]);
+  }
+  return a[0];
 }
 
-// One wave per strip (reduced dim contiguous). For argmax/argmin each lane
-// tracks the first winner of its own positions among non-NaN values; a NaN
-// at position 0 forces index 0, matching the sequential scan.
-template <int K>
-__global__ __launch_bounds__(BS) void reduce_contig_k(const float* __restrict__ x, RPlan p, int64_t nout,
-                                                      float* __restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const int64_t e = ((int64_t)blockIdx.x * BS + threadIdx.x) >> 6;
-  if (e >= nout) return;
+// A strip per group of TPS threads.
+template <int K, int TPS>
+__global__ __launch_bounds__((TPS > BS ? TPS : BS)) void reduce_contig_k(const float* __restrict__ x, RPlan p,
+                                                                         int64_t nout, float* __restrict__ out) {
+  constexpr int NT = TPS > BS ? TPS : BS;
+  __shared__ Part<K> lds[TPS / 64];
+  const int t = threadIdx.x % TPS;
+  const int64_t e = (int64_t)blockIdx.x * (NT / TPS) + threadIdx.x / TPS;
+  if (e >= nout) return;  // TPS > 64: one strip per block, the whole block leaves together
   const float* s = x + base_of(p, e);
-  const int64_t len = p.len;
-  float v;
-  int64_t idx = 0;
-  bool has = false;
-  if constexpr (K == OXI_REDUCE_MAX) v = -__builtin_huge_valf();
-  else if constexpr (K == OXI_REDUCE_MIN) v = __builtin_huge_valf();
-  else v = 0.f;
-  for (int64_t k = lane; k < len; k += 64) {
-    const float a = s[k];
-    if constexpr (K == OXI_REDUCE_SUM || K == OXI_REDUCE_MEAN) v += a;
-    else if constexpr (K == OXI_REDUCE_NORM) v += a * a;
-    else if constexpr (K == OXI_REDUCE_MAX) v = fmaxf(v, a);
-    else if constexpr (K == OXI_REDUCE_MIN) v = fminf(v, a);
-    else {
-      if (a == a) {
-        const bool better = (K == OXI_REDUCE_ARGMAX) ? (a > v) : (a < v);
-        if (!has || better) { v = a; idx = k; has = true; }
-      }
-    }
-  }
+  const Part<K> a = strip_part<K, TPS>(s, 0, p.len, t, lds);
+  if (t == 0) out[e] = strip_result<K>(s, a, p.len);
+}
+
+// Few long strips: block (e, j) leaves the state of positions
+// [j * part, (j + 1) * part) of strip e; strip_finish_k merges a strip's
+// parts, sums in float64.
+template <int K>
+__global__ __launch_bounds__(BS) void reduce_parts_k(const float* __restrict__ x, RPlan p, int64_t part, int parts,
+                                                     Part<K>* __restrict__ ws) {
+  __shared__ Part<K> lds[BS / 64];
+  const int64_t e = blockIdx.x / parts;
+  const int64_t k0 = (int64_t)(blockIdx.x % parts) * part;
+  const Part<K> a = strip_part<K, BS>(x + base_of(p, e), k0, min<int64_t>(k0 + part, p.len), threadIdx.x, lds);
+  if (threadIdx.x == 0) ws[blockIdx.x] = a;
+}
+
+template <int K>
+__global__ __launch_bounds__(64) void strip_finish_k(const float* __restrict__ x, RPlan p, int parts,
+                                                     const Part<K>* __restrict__ ws, float* __restrict__ out) {
+  const int64_t e = blockIdx.x;
+  const Part<K>* w = ws + e * parts;
+  const int t = threadIdx.x;
+  Part<K> a = Part<K>::none();
+  if constexpr (is_fold(K)) {
+    double d = 0.0;
+    for (int j = t; j < parts; j += 64) d += (double)w[j].v;
+    d = wave_sum(d);
+    a.v = (float)d;
+  } else {
+    for (int j = t; j < parts; j += 64) a.merge(w[j]);
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    const float vo = __shfl_xor(v, m, 64);
-    const int64_t io = __shfl_xor(idx, m, 64);
-    const bool ho = __shfl_xor((int)has, m, 64) != 0;
-    combine<K>(v, idx, has, vo, io, ho);
+    for (int m = 32; m >= 1; m >>= 1) a.merge(part_xor<K>(a, m));
   }
-  if (lane == 0) {
-    float r;
-    if constexpr (K == OXI_REDUCE_MEAN) r = v / (float)len;
-    else if constexpr (K == OXI_REDUCE_NORM) r = sqrtf(v);
-    else if constexpr (K == OXI_REDUCE_ARGMAX || K == OXI_REDUCE_ARGMIN) r = (s[0] != s[0] || !has) ? 0.f : (float)idx;
-    else r = v;
-    out[e] = r;
-  }
+  if (t == 0) out[e] = strip_result<K>(x + base_of(p, e), a, p.len);
+}
+
+// Whether the library stream is being captured into a graph: a launch that
+// needs a workspace then takes the route without one (the block would go back
+// to the allocator when the call returns, and be written again by a replay).
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
 
 template <int K>
 int launch(const float* x, const RPlan& p, int64_t nout, float* out) {
   hipStream_t s = stream();
   if (p.rst == 1 && p.len >= 32) {
-    const int64_t blocks = ceil_div(nout * 64, BS);
+    if (nout < cu_count() && p.len >= SPLIT_MIN_LEN && !capturing(s)) {
+      const int64_t want = ceil_div(SPLIT_BLOCKS_PER_CU * (int64_t)cu_count(), nout);
+      int64_t part = ceil_div(ceil_div(p.len, want), SPLIT_MIN_PART) * SPLIT_MIN_PART;
+      const int64_t parts = ceil_div(p.len, part);
+      Workspace ws(sizeof(Part<K>) * (size_t)(nout * parts));
+      if (ws.p) {  // else: the one-launch route below
+        reduce_parts_k<K><<<dim3((unsigned)(nout * parts)), dim3(BS), 0, s>>>(x, p, part, (int)parts, ws.as<Part<K>>());
+        if (int rc = check_launch("reduce")) return rc;
+        strip_finish_k<K><<<dim3((unsigned)nout), dim3(64), 0, s>>>(x, p, (int)parts, ws.as<Part<K>>(), out);
+        return check_launch("reduce_finish");
+      }
+    }
+    const int tps = p.len <= WAVE_MAX_LEN ? 64 : nout < 2 * cu_count() ? 1024 : 256;
+    const int64_t blocks = tps == 64 ? ceil_div(nout * 64, BS) : nout;
     if (blocks < ((int64_t)1 << 31)) {
-      reduce_contig_k<K><<<dim3((unsigned)blocks), dim3(BS), 0, s>>>(x, p, nout, out);
+      const dim3 g((unsigned)blocks);
+      if (tps == 64) reduce_contig_k<K, 64><<<g, dim3(BS), 0, s>>>(x, p, nout, out);
+      else if (tps == 256) reduce_contig_k<K, 256><<<g, dim3(256), 0, s>>>(x, p, nout, out);
+      else reduce_contig_k<K, 1024><<<g, dim3(1024), 0, s>>>(x, p, nout, out);
       return check_launch("reduce");
     }
   }
-  if constexpr (K != OXI_REDUCE_ARGMAX && K != OXI_REDUCE_ARGMIN) {
-    // vector path: innermost remaining dim contiguous, every row start 16-byte aligned
-    bool vec = p.nd > 0 && p.st[p.nd - 1] == 1 && p.size[p.nd - 1] % 4 == 0 && p.rst % 4 == 0 &&
-               (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
-    for (int d = 0; d + 1 < p.nd && vec; ++d)
-      if (p.st[d] % 4) vec = false;
-    if (vec) {
+  const bool unit = p.nd > 0 && p.st[p.nd - 1] == 1;  // outputs adjacent in memory
+  // vector path: every row start 16-byte aligned
+  bool vec = unit && p.size[p.nd - 1] % 4 == 0 && p.rst % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+  for (int d = 0; d + 1 < p.nd && vec; ++d)
+    if (p.st[d] % 4) vec = false;
+  if (unit && p.len >= COLS_MIN_LEN && nout <= COLS_MAX_OUT) {
+    const int64_t inner = p.size[p.nd - 1];
+    const int64_t groups = ceil_div(inner, COLS_C);
+    const dim3 g((unsigned)(nout / inner * groups));
+    if (vec) reduce_cols_k<K, true><<<g, dim3(COLS_NT), 0, s>>>(x, p, inner, groups, out);
+    else reduce_cols_k<K, false><<<g, dim3(COLS_NT), 0, s>>>(x, p, inner, groups, out);
+    return check_launch("reduce");
+  }
+  if constexpr (!is_arg(K)) {
+    if (vec && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
       const int64_t nout4 = nout / 4;
       const int64_t blocks = std::min<int64_t>(ceil_div(nout4, BS), (int64_t)cu_count() * 64);
       reduce_strided_vec_k<K><<<dim3((unsigned)std::max<int64_t>(blocks, 1)), dim3(BS), 0, s>>>(x, p, nout4, out);

@@ -14,6 +14,9 @@
 namespace oxi {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+// A float4 at any float address. gfx950 does unaligned global accesses, so a
+// load or store of one is still a single 16-byte instruction.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
 // Streaming accesses: each tensor byte crosses memory once per kernel.
 // Loads are non-temporal (a one-pass stream should not evict what the next
