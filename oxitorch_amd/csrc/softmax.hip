@@ -14,6 +14,7 @@
 // writes (softmax - onehot) * g / n. Bytes per row: 1 read fwd, 1 read + 1
 // write bwd, instead of the reference's dense one-hot and ~16 passes
 // (python/oxitorch/nn/functional.py:277-293).
+#include <algorithm>
 #include <cmath>
 
 #include "internal.h"
@@ -53,7 +54,7 @@ template <int TPR>
 __device__ __forceinline__ void group_online(Online& o, float* lds) {
   const float M = group_max<TPR>(o.m, lds);
   float part = (o.m == NEG_INF) ? ((o.s != o.s) ? o.s : 0.f) : o.s * expf(o.m - M);
-  const float S = group_sum<TPR, float>(part, lds + BS / 64);
+  const float S = group_sum<TPR, float>(part, lds + TPR / 64);
   o.m = M;
   o.s = S;
 }
@@ -216,15 +217,19 @@ __device__ __forceinline__ f4 drop_lane(const f4& v, int j) {
   return f4{j == 0 ? P : v.x, j == 1 ? P : v.y, j == 2 ? P : v.z, j == 3 ? P : v.w};
 }
 
-// Rows longer than the register-row kernel takes (more than 16384 float4s,
-// or not vectorizable): one block per row, streaming it.
+// Rows the register-row kernel does not take (more than 16384 float4s, or not
+// a multiple of 4 classes at a 16-byte address): one block per row, streaming
+// it with CE_U float4s in flight a thread, at whatever float alignment the row
+// has, and the last C % 4 logits on their own. HBM bounds it: 4096 rows of
+// 50257 classes take 136-160 us (5.1-6.0 TB/s) where single floats took 330.
 // lse[row] = max + log(sum exp(x - max));
 // picked[row] = (x[t] - max) - log(sum)  (the reference's ls[row, t]), or
 // NaN where the reference's one-hot product makes it NaN (onehot_nan).
-__global__ __launch_bounds__(CE_BS) void ce_fwd_k(const float* __restrict__ logits, const int64_t* __restrict__ targets,
-                                                  float* __restrict__ lse, float* __restrict__ picked, int64_t n, int C,
-                                                  int vec, int* __restrict__ guard) {
-  __shared__ float lds[2 * (CE_BS / 64)];
+template <int NT>
+__global__ __launch_bounds__(NT) void ce_fwd_k(const float* __restrict__ logits, const int64_t* __restrict__ targets,
+                                               float* __restrict__ lse, float* __restrict__ picked, int64_t n, int C,
+                                               int* __restrict__ guard) {
+  __shared__ float lds[2 * (NT / 64)];
   const int64_t row = blockIdx.x;
   const float* xr = logits + row * C;
   int64_t tg = targets[row];
@@ -232,49 +237,47 @@ __global__ __launch_bounds__(CE_BS) void ce_fwd_k(const float* __restrict__ logi
   if (bad) tg = 0;
   float mn = -NEG_INF;
   Online o;
-  if (vec) {
-    const f4* p = reinterpret_cast<const f4*>(xr);
-    const int c4 = C >> 2;
-    const int ct = (int)(tg >> 2);
-    const int jt = (int)(tg & 3);
-    int c = threadIdx.x;
-    for (; c + (CE_U - 1) * CE_BS < c4; c += CE_U * CE_BS) {
-      f4 v[CE_U];
+  const f4u* p = reinterpret_cast<const f4u*>(xr);
+  const int c4 = C >> 2;
+  const int ct = (int)(tg >> 2);
+  const int jt = (int)(tg & 3);
+  int c = threadIdx.x;
+  for (; c + (CE_U - 1) * NT < c4; c += CE_U * NT) {
+    f4 v[CE_U];
 #pragma unroll
-      for (int u = 0; u < CE_U; ++u) v[u] = ld_stream(p + c + u * CE_BS);
+    for (int u = 0; u < CE_U; ++u) v[u] = ld_stream(p + c + u * NT);
 #pragma unroll
-      for (int u = 0; u < CE_U; ++u) mn = fminf(mn, min4(c + u * CE_BS == ct ? drop_lane(v[u], jt) : v[u]));
-      float cm = max4(v[0]);
+    for (int u = 0; u < CE_U; ++u) mn = fminf(mn, min4(c + u * NT == ct ? drop_lane(v[u], jt) : v[u]));
+    float cm = max4(v[0]);
 #pragma unroll
-      for (int u = 1; u < CE_U; ++u) cm = fmaxf(cm, max4(v[u]));
-      if (cm > o.m) {
-        o.s = (o.m == NEG_INF) ? 0.f : o.s * expf(o.m - cm);
-        o.m = cm;
-      }
-      if (o.m != NEG_INF) {
-        float acc = 0.f;
-#pragma unroll
-        for (int u = 0; u < CE_U; ++u) acc += sum4(exp4(v[u] - o.m));
-        o.s += acc;
-      } else {
-#pragma unroll
-        for (int u = 0; u < CE_U; ++u) o.add4(v[u]);
-      }
+    for (int u = 1; u < CE_U; ++u) cm = fmaxf(cm, max4(v[u]));
+    if (cm > o.m) {
+      o.s = (o.m == NEG_INF) ? 0.f : o.s * expf(o.m - cm);
+      o.m = cm;
     }
-    for (; c < c4; c += CE_BS) {
-      const f4 v = p[c];
-      o.add4(v);
-      mn = fminf(mn, min4(c == ct ? drop_lane(v, jt) : v));
-    }
-  } else {
-    for (int c = threadIdx.x; c < C; c += CE_BS) {
-      const float v = xr[c];
-      o.add1(v);
-      if (c != tg) mn = fminf(mn, v);
+    if (o.m != NEG_INF) {
+      float acc = 0.f;
+#pragma unroll
+      for (int u = 0; u < CE_U; ++u) acc += sum4(exp4(v[u] - o.m));
+      o.s += acc;
+    } else {
+#pragma unroll
+      for (int u = 0; u < CE_U; ++u) o.add4(v[u]);
     }
   }
-  group_online<CE_BS>(o, lds);
-  mn = -group_max<CE_BS>(-mn, lds);
+  for (; c < c4; c += NT) {
+    const f4 v = p[c];
+    o.add4(v);
+    mn = fminf(mn, min4(c == ct ? drop_lane(v, jt) : v));
+  }
+  if ((int)threadIdx.x < (C & 3)) {
+    const int e = 4 * c4 + threadIdx.x;
+    const float v = xr[e];
+    o.add1(v);
+    if (e != tg) mn = fminf(mn, v);
+  }
+  group_online<NT>(o, lds);
+  mn = -group_max<NT>(-mn, lds);
   if (threadIdx.x == 0) {
     if (bad) atomicOr(guard, 1);
     const float L = logf(o.s);
@@ -454,14 +457,29 @@ __global__ __launch_bounds__(CE_BS) void ce_bwd_k(const float* __restrict__ logi
       }
     }
   } else {
-    const int per_block = CE_BS * CE_BU;
-    const int c0 = blockIdx.x * per_block + threadIdx.x;
-    for (int u = 0; u < CE_BU; ++u) {
-      const int c = c0 + u * CE_BS;
-      if (c < C) {
-        float e = expf(xr[c] - l);
-        if (c == t) e -= 1.f;
-        dr[c] = e * scale;
+    // Rows at any float alignment: the gradient's 16-byte granules, whole in
+    // the row, are a float4 each (the logits' share their phase unless the
+    // buffers differ in it); the up to 3 classes before the first and after
+    // the last go one each to the first block's threads. (4096, 50257) takes
+    // 264-275 us (6.0-6.2 TB/s) where a float a thread took 550.
+    const int head = min((int)((0 - (reinterpret_cast<uintptr_t>(dr) >> 2)) & 3u), C);
+    const int c4 = (C - head) >> 2;
+    const int c = blockIdx.x * CE_BS + threadIdx.x;
+    if (c < c4) {
+      const int e0 = head + 4 * c;
+      f4 e = exp4(ld_stream(reinterpret_cast<const f4u*>(xr + e0)) - l);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (e0 + j == t) e[j] -= 1.f;
+      st_stream<NTS>(e * scale, reinterpret_cast<f4*>(dr + e0));
+    }
+    if (blockIdx.x == 0 && threadIdx.x < 6) {
+      const int k = threadIdx.x;
+      const int e0 = k < 3 ? k : head + 4 * c4 + (k - 3);
+      if (k < 3 ? e0 < head : e0 < C) {
+        float e = exp_le0(xr[e0] - l);
+        if (e0 == t) e -= 1.f;
+        dr[e0] = e * scale;
       }
     }
   }
@@ -672,7 +690,11 @@ int ce_forward(const char* what, const float* logits, const int64_t* targets, fl
 #undef OXI_CE_ROWS
 #undef OXI_CE_GO
     default:
-      ce_fwd_k<<<grid, dim3(CE_BS), 0, stream()>>>(logits, targets, lse, pk, n, (int)c, vec, guard_flag());
+      // fewer rows than two a CU: 1024 threads to a long row
+      if (n < 2 * cu_count() && c > 16384)
+        ce_fwd_k<1024><<<grid, dim3(1024), 0, stream()>>>(logits, targets, lse, pk, n, (int)c, guard_flag());
+      else
+        ce_fwd_k<CE_BS><<<grid, dim3(CE_BS), 0, stream()>>>(logits, targets, lse, pk, n, (int)c, guard_flag());
   }
   if (int rc = check_launch(what)) return rc;
   ce_mean_k<<<1, 1024, 0, stream()>>>(picked.as<float>(), n, loss);
@@ -704,7 +726,7 @@ int oxi_cross_entropy_bwd(const float* logits, const int64_t* targets, const flo
     return fail(OXI_INVALID_ARGUMENT, "cross_entropy_bwd: NULL tensor pointer");
   OXI_CHECK_INIT();
   const int vec = (c % 4 == 0 && aligned16({logits, dlogits})) ? 1 : 0;
-  const int64_t units = vec ? c / 4 : c;
+  const int64_t units = std::max<int64_t>(1, c / 4);  // at least one block a row
   const unsigned gx = (unsigned)ceil_div(units, CE_BS * CE_BU);
   const bool nts = nt_stores(n * c * 4);
   if (n > 65535) {
