@@ -5,7 +5,8 @@
 // row per row group with the row held in registers when it fits
 // (len <= 8192, 16-byte aligned), so x is read once and y written once;
 // longer rows stream twice (online max/sum pass, then the write pass).
-// inner > 1 runs one thread per (outer, inner) column, coalesced across inner.
+// inner > 1 runs tiles of adjacent columns, their positions spread over the
+// block and held in registers.
 //
 // Cross-entropy (mean reduction) is fused into two kernels: the forward streams
 // each logits row once with an online (max, sum-exp) and writes the row's
@@ -159,41 +160,256 @@ __global__ __launch_bounds__(BS) void sm_bwd_loop_k(const float* __restrict__ y,
 }
 
 // ---------------------------------------------------------------------------
-// Middle-dim kernels (inner > 1): one thread per (o, i) column.
+// Middle-dim kernels (inner > 1). A block owns TX units of W adjacent columns
+// (4, or single columns when inner < 4) and spreads their len positions over
+// TY threads a unit, NV positions a thread: up to TY * NV positions are held
+// in registers, so x crosses HBM once and the columns' maxima and sums are
+// combined through LDS; longer columns (NV = 0) are streamed twice, MID_U
+// positions in flight a thread, with an online maximum and sum. HBM bounds
+// both. A row's last unit starts at inner - W, so it may repeat columns of the
+// one before: both form and write the same values. TX and TY are chosen on the
+// host (mid_shape): wide tiles for few positions, 128 bytes of a row (TX = 8)
+// for many. Against one thread a column walking it twice, the log-softmax of
+// (16, 150, 4096) takes 14.6 us forward (5.4 TB/s) and 20.4 us backward
+// instead of 115 and 92, of (2, 2846, 1901), streamed, 73 and 59 instead of
+// 1800 and 1500, of (65536, 8, 3) 7.7 and 8.4 instead of 8.9 and 9.8. Plain
+// loads: a row's 128-byte lines are shared by tiles when inner is odd, and
+// non-temporal ones took 21 and 27 us at (16, 150, 4096) with the input in the
+// Infinity Cache (from HBM: 45.6 us for both against 48.0). 12 positions a
+// thread instead of 8: 15.7 against 21.2 us there with those loads, and slower
+// below 64 positions.
 
-template <bool LOG>
-__global__ __launch_bounds__(BS) void sm_fwd_col_k(const float* __restrict__ x, float* __restrict__ y,
-                                                   int64_t outer, int64_t len, int64_t inner) {
-  const int64_t id = (int64_t)blockIdx.x * BS + threadIdx.x;
-  if (id >= outer * inner) return;
-  const int64_t o = id / inner, i = id % inner;
-  const float* xc = x + o * len * inner + i;
-  float* yc = y + o * len * inner + i;
-  Online st;
-  for (int64_t k = 0; k < len; ++k) st.add1(xc[k * inner]);
-  const float L = logf(st.s);
-  for (int64_t k = 0; k < len; ++k) {
-    const float z = xc[k * inner] - st.m;
-    yc[k * inner] = LOG ? z - L : expf(z) / st.s;
+constexpr int MID_U = 4;
+
+template <int W>
+struct Lanes {  // W columns' values
+  typedef float type __attribute__((ext_vector_type(W), aligned(4)));
+};
+template <>
+struct Lanes<1> {
+  typedef float type;
+};
+
+// The unit of this thread.
+struct MidUnit {
+  int tx, ty;     // its place in the block's tile
+  bool act;       // it has positions of an existing unit
+  int64_t base;   // its first column's position 0
+};
+
+// Unit id: the units of every outer index, one after another.
+template <int W>
+__device__ __forceinline__ MidUnit mid_unit(int64_t len, int64_t inner, int64_t units, int64_t total, int TX) {
+  MidUnit m;
+  m.tx = threadIdx.x % TX;
+  m.ty = threadIdx.x / TX;
+  const int64_t id = (int64_t)blockIdx.x * TX + m.tx;
+  m.act = id < total;
+  const int64_t o = id / units, u = id % units;
+  m.base = o * len * inner + min<int64_t>(u * W, inner - W);
+  return m;
+}
+
+// op over the TY threads of every unit; each gets the result. `red` holds a
+// value per thread and is free again after the call.
+template <class V, class Op>
+__device__ __forceinline__ V mid_combine(V v, V* red, const MidUnit& m, int TX, int TY, Op op) {
+  if (TY == 1) return v;
+  red[m.ty * TX + m.tx] = v;
+  for (int h = TY >> 1; h >= 1; h >>= 1) {  // TY is a power of two
+    __syncthreads();
+    if (m.ty < h) red[m.ty * TX + m.tx] = op(red[m.ty * TX + m.tx], red[(m.ty + h) * TX + m.tx]);
+  }
+  __syncthreads();
+  v = red[m.tx];
+  __syncthreads();
+  return v;
+}
+
+template <int W>
+__device__ __forceinline__ float& at(typename Lanes<W>::type& v, int j) {
+  return reinterpret_cast<float*>(&v)[j];
+}
+
+template <bool LOG, int W, int NV, int NT>
+__global__ __launch_bounds__(NT) void sm_fwd_mid_k(const float* __restrict__ x, float* __restrict__ y, int64_t len,
+                                                   int64_t inner, int64_t units, int64_t total, int TX, int TY) {
+  using V = typename Lanes<W>::type;
+  constexpr int N = NV ? NV : MID_U;
+  __shared__ V red[NT];
+  const MidUnit u = mid_unit<W>(len, inner, units, total, TX);
+  const float* xc = x + u.base;
+  float* yc = y + u.base;
+  auto each = [](auto f) {
+#pragma unroll
+    for (int j = 0; j < W; ++j) f(j);
+  };
+  auto vmax = [&](V a, V b) {
+    each([&](int j) { at<W>(a, j) = fmaxf(at<W>(a, j), at<W>(b, j)); });
+    return a;
+  };
+  auto vsum = [](V a, V b) { return a + b; };
+  V v[N];
+  // positions k0 + ty, + TY, ...: those past the end give -inf, which counts for nothing
+  auto load = [&](int64_t k0) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int64_t k = k0 + u.ty + (int64_t)i * TY;
+      each([&](int j) { at<W>(v[i], j) = NEG_INF; });
+      if (u.act && k < len) v[i] = *reinterpret_cast<const V*>(xc + k * inner);
+    }
+  };
+  V m, s;
+  each([&](int j) {
+    at<W>(m, j) = NEG_INF;
+    at<W>(s, j) = 0.f;
+  });
+  if constexpr (NV > 0) {
+    load(0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) m = vmax(m, v[i]);
+  } else {
+    for (int64_t k0 = 0; k0 < len; k0 += (int64_t)N * TY) {
+      load(k0);
+      each([&](int j) {
+        float cm = at<W>(m, j);
+#pragma unroll
+        for (int i = 0; i < N; ++i) cm = fmaxf(cm, at<W>(v[i], j));
+        const float ref = cm == NEG_INF ? 0.f : cm;
+        float acc = at<W>(s, j) * exp_le0(at<W>(m, j) - ref);
+#pragma unroll
+        for (int i = 0; i < N; ++i) acc += exp_le0(at<W>(v[i], j) - ref);
+        at<W>(s, j) = acc;
+        at<W>(m, j) = cm;
+      });
+    }
+  }
+  const V M = mid_combine(m, red, u, TX, TY, vmax);
+  if constexpr (NV > 0) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (u.ty + (int64_t)i * TY < len)
+        each([&](int j) {
+          V Mv = M;
+          const float z = at<W>(v[i], j) - at<W>(Mv, j);
+          const float e = exp_le0(z);
+          at<W>(s, j) += e;
+          at<W>(v[i], j) = LOG ? z : e;
+        });
+  } else {
+    each([&](int j) {
+      V Mv = M;
+      const float ref = at<W>(Mv, j) == NEG_INF ? 0.f : at<W>(Mv, j);
+      at<W>(s, j) *= exp_le0(at<W>(m, j) - ref);
+    });
+  }
+  V S = mid_combine(s, red, u, TX, TY, vsum);
+  V out;
+  auto finish = [&](V e) {  // from z or e (NV > 0), or from x
+    V Mv = M;
+    each([&](int j) {
+      if constexpr (NV == 0) {
+        const float z = at<W>(e, j) - at<W>(Mv, j);
+        at<W>(out, j) = LOG ? z - logf(at<W>(S, j)) : exp_le0(z) / at<W>(S, j);
+      } else {
+        at<W>(out, j) = LOG ? at<W>(e, j) - at<W>(S, j) : at<W>(e, j) / at<W>(S, j);
+      }
+    });
+    return out;
+  };
+  if (!u.act) return;
+  if constexpr (NV > 0) {
+    if constexpr (LOG) each([&](int j) { at<W>(S, j) = logf(at<W>(S, j)); });
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int64_t k = u.ty + (int64_t)i * TY;
+      if (k < len) *reinterpret_cast<V*>(yc + k * inner) = finish(v[i]);
+    }
+  } else {
+    for (int64_t k0 = u.ty; k0 < len; k0 += (int64_t)N * TY) {
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if (k0 + (int64_t)i * TY < len) v[i] = *reinterpret_cast<const V*>(xc + (k0 + (int64_t)i * TY) * inner);
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if (k0 + (int64_t)i * TY < len) *reinterpret_cast<V*>(yc + (k0 + (int64_t)i * TY) * inner) = finish(v[i]);
+    }
   }
 }
 
-template <bool LOG>
-__global__ __launch_bounds__(BS) void sm_bwd_col_k(const float* __restrict__ y, const float* __restrict__ g,
-                                                   float* __restrict__ dx, int64_t outer, int64_t len, int64_t inner) {
-  const int64_t id = (int64_t)blockIdx.x * BS + threadIdx.x;
-  if (id >= outer * inner) return;
-  const int64_t o = id / inner, i = id % inner;
-  const int64_t base = o * len * inner + i;
-  float s = 0.f;
-  for (int64_t k = 0; k < len; ++k) {
-    const int64_t p = base + k * inner;
-    s += LOG ? g[p] : g[p] * y[p];
+template <bool LOG, int W, int NV, int NT>
+__global__ __launch_bounds__(NT) void sm_bwd_mid_k(const float* __restrict__ y, const float* __restrict__ g,
+                                                   float* __restrict__ dx, int64_t len, int64_t inner, int64_t units,
+                                                   int64_t total, int TX, int TY) {
+  using V = typename Lanes<W>::type;
+  constexpr int N = NV ? NV : MID_U;
+  __shared__ V red[NT];
+  const MidUnit u = mid_unit<W>(len, inner, units, total, TX);
+  const float *yc = y + u.base, *gc = g + u.base;
+  float* dc = dx + u.base;
+  V a[N], b[N];  // y and g; 0 past the end
+  auto load = [&](int64_t k0) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int64_t k = k0 + u.ty + (int64_t)i * TY;
+      a[i] = V{};
+      b[i] = V{};
+      if (u.act && k < len) {
+        a[i] = *reinterpret_cast<const V*>(yc + k * inner);
+        b[i] = *reinterpret_cast<const V*>(gc + k * inner);
+      }
+    }
+  };
+  V s = V{};
+  for (int64_t k0 = 0; k0 < len; k0 += (int64_t)N * TY) {
+    load(k0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) s = s + (LOG ? b[i] : b[i] * a[i]);
+    if constexpr (NV > 0) break;
   }
-  for (int64_t k = 0; k < len; ++k) {
-    const int64_t p = base + k * inner;
-    dx[p] = LOG ? g[p] - expf(y[p]) * s : y[p] * (g[p] - s);
+  const V S = mid_combine(s, red, u, TX, TY, [](V p, V q) { return p + q; });
+  if (!u.act) return;
+  for (int64_t k0 = 0; k0 < len; k0 += (int64_t)N * TY) {
+    if constexpr (NV == 0) load(k0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int64_t k = k0 + u.ty + (int64_t)i * TY;
+      if (k >= len) continue;
+      V o;
+      if constexpr (LOG) {
+#pragma unroll
+        for (int j = 0; j < W; ++j) at<W>(o, j) = exp_le0(at<W>(a[i], j));
+        o = b[i] - o * S;
+      } else {
+        o = a[i] * (b[i] - S);
+      }
+      *reinterpret_cast<V*>(dc + k * inner) = o;
+    }
+    if constexpr (NV > 0) break;
   }
+}
+
+// The launch of a middle-dim kernel: NT threads, TX units by TY positions a
+// block (TX * TY = NT), NV positions a thread (0: streamed).
+struct MidShape {
+  int nt, tx, ty, nv;
+  int64_t units, total, blocks;
+};
+
+MidShape mid_shape(int64_t outer, int64_t len, int64_t inner) {
+  MidShape m;
+  const int w = inner >= 4 ? 4 : 1;
+  const int nv = w == 4 ? 8 : 16;  // positions a thread holds at most
+  m.units = ceil_div(inner, w);
+  m.total = outer * m.units;
+  m.nt = len <= 32 * nv ? 256 : 1024;
+  m.ty = 1;
+  while ((int64_t)m.ty * nv < len && m.ty < m.nt / 8) m.ty <<= 1;
+  m.tx = m.nt / m.ty;
+  const int64_t per = ceil_div(len, m.ty);
+  m.nv = per <= nv / 4 ? nv / 4 : per <= nv ? nv : 0;
+  m.blocks = ceil_div(m.total, m.tx);
+  return m;
 }
 
 // ---------------------------------------------------------------------------
@@ -509,6 +725,23 @@ int check_olen(const char* what, int64_t outer, int64_t len, int64_t inner, std:
   return OXI_OK;
 }
 
+#define OXI_MID_GO(K, W, NV, NT, ...)                                                                       \
+  K<LOG, W, NV, NT><<<dim3((unsigned)m.blocks), dim3(NT), 0, s>>>(__VA_ARGS__, len, inner, m.units, m.total,   \
+                                                                 m.tx, m.ty)
+#define OXI_MID_NT(K, W, NV, ...)                                                                           \
+  if (m.nt == 256) OXI_MID_GO(K, W, NV, 256, __VA_ARGS__);                                                  \
+  else OXI_MID_GO(K, W, NV, 1024, __VA_ARGS__);
+#define OXI_MID(K, ...)                                                                                     \
+  if (inner >= 4) {                                                                                         \
+    if (m.nv == 2) { OXI_MID_NT(K, 4, 2, __VA_ARGS__) }                                                     \
+    else if (m.nv == 8) { OXI_MID_NT(K, 4, 8, __VA_ARGS__) }                                                \
+    else { OXI_MID_NT(K, 4, 0, __VA_ARGS__) }                                                               \
+  } else {                                                                                                  \
+    if (m.nv == 4) { OXI_MID_NT(K, 1, 4, __VA_ARGS__) }                                                     \
+    else if (m.nv == 16) { OXI_MID_NT(K, 1, 16, __VA_ARGS__) }                                              \
+    else { OXI_MID_NT(K, 1, 0, __VA_ARGS__) }                                                               \
+  }
+
 template <bool LOG>
 int launch_fwd(const float* x, float* y, int64_t outer, int64_t len, int64_t inner) {
   hipStream_t s = stream();
@@ -543,7 +776,8 @@ int launch_fwd(const float* x, float* y, int64_t outer, int64_t len, int64_t inn
 #undef OXI_SMF
 #undef OXI_SMF_GO
   } else {
-    sm_fwd_col_k<LOG><<<dim3((unsigned)ceil_div(outer * inner, BS)), dim3(BS), 0, s>>>(x, y, outer, len, inner);
+    const MidShape m = mid_shape(outer, len, inner);
+    OXI_MID(sm_fwd_mid_k, x, y)
   }
   return check_launch(LOG ? "log_softmax_fwd" : "softmax_fwd");
 }
@@ -582,7 +816,8 @@ int launch_bwd(const float* y, const float* g, float* dx, int64_t outer, int64_t
 #undef OXI_SMB
 #undef OXI_SMB_GO
   } else {
-    sm_bwd_col_k<LOG><<<dim3((unsigned)ceil_div(outer * inner, BS)), dim3(BS), 0, s>>>(y, g, dx, outer, len, inner);
+    const MidShape m = mid_shape(outer, len, inner);
+    OXI_MID(sm_bwd_mid_k, y, g, dx)
   }
   return check_launch(LOG ? "log_softmax_bwd" : "softmax_bwd");
 }
