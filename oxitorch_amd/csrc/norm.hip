@@ -42,29 +42,33 @@ __device__ __forceinline__ float rsum1(float v, float* lds) { return group_sum_o
 // ---------------------------------------------------------------------------
 // Forward, register-resident rows.
 
-// FULL: rows of exactly TPR * NV float4s (H = 4 * TPR * NV), a compile-time
-// row length: no padding lanes, no bounds checks.
+// KIND: RowKind; ROW_FULL rows have a compile-time length, no padding lanes and
+// no bounds checks.
 // NT: threads per block, row_block_threads(TPR) or, for one-wave rows, 1024.
-template <int TPR, int NV, bool LN, bool NTS, bool FULL, int NT>
+template <int TPR, int NV, bool LN, bool NTS, int KIND, int NT>
 __global__ __launch_bounds__(NT) void norm_fwd_k(const float* __restrict__ x, const float* __restrict__ w,
                                                  const float* __restrict__ b, float* __restrict__ y,
                                                  float* __restrict__ mean, float* __restrict__ rstd,
                                                  int64_t rows, int H_arg, float eps) {
-  const int H = FULL ? 4 * TPR * NV : H_arg;
+  const int H = KIND == ROW_FULL ? 4 * TPR * NV : H_arg;
   constexpr int GPB = NT / TPR;
   __shared__ float lds[2 * (NT / 64)];  // mean, then variance
   const int t = threadIdx.x % TPR;
   const int64_t row = (int64_t)blockIdx.x * GPB + threadIdx.x / TPR;
   if (row >= rows) return;  // GPB == 1 whenever TPR > 64: the whole block leaves together
-  const int h4 = H >> 2;
+  const int h4 = row_slots<KIND>(H);
   const float fH = (float)H;
   RowTile<TPR, NV> xt;
-  xt.load(x + row * H, h4, t);
+  if constexpr (KIND == ROW_ODD) xt.load_odd(x + row * H, H, h4, t);
+  else xt.load(x + row * H, h4, t);
   float mu = 0.f;
   if constexpr (LN) {
     float s = 0.f;
 #pragma unroll
-    for (int k = 0; k < NV; ++k) s += (xt.v[k].x + xt.v[k].y) + (xt.v[k].z + xt.v[k].w);
+    for (int k = 0; k < NV; ++k) {
+      const f4 v = without_dup<KIND>(xt.v[k], H, k * TPR + t);
+      s += (v.x + v.y) + (v.z + v.w);
+    }
     mu = rsum1<TPR>(s, lds) / fH;
 #pragma unroll
     for (int k = 0; k < NV; ++k)
@@ -73,7 +77,7 @@ __global__ __launch_bounds__(NT) void norm_fwd_k(const float* __restrict__ x, co
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const f4 v = xt.v[k];
+    const f4 v = without_dup<KIND>(xt.v[k], H, k * TPR + t);
     ss += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
   }
   const float var = rsum1<TPR>(ss, lds + NT / 64) / fH;
@@ -89,15 +93,22 @@ __global__ __launch_bounds__(NT) void norm_fwd_k(const float* __restrict__ x, co
     const int c = k * TPR + t;
     if (c < h4) {
       f4 o = xt.v[k] * inv;
-      if (w) o = o * w4[c];
-      if (LN && b) o = o + b4[c];
+      if constexpr (KIND == ROW_ODD) {
+        if (w) o = o * ld_odd(w, H, c);
+        if (LN && b) o = o + ld_odd(b, H, c);
+      } else {
+        if (w) o = o * w4[c];
+        if (LN && b) o = o + b4[c];
+      }
       xt.v[k] = o;
     }
   }
-  xt.template store<NTS>(y + row * H, h4, t);
+  if constexpr (KIND == ROW_ODD) xt.store_odd(y + row * H, H, h4, t);
+  else xt.template store<NTS>(y + row * H, h4, t);
 }
 
-// Forward for any H / alignment: one block per row, rows re-read from cache.
+// Forward for rows of fewer than 4 floats or more than the register kernels
+// take: one block per row, rows re-read from cache.
 template <bool LN>
 __global__ __launch_bounds__(BS) void norm_fwd_loop_k(const float* __restrict__ x, const float* __restrict__ w,
                                                       const float* __restrict__ b, float* __restrict__ y,
@@ -138,15 +149,15 @@ __global__ __launch_bounds__(BS) void norm_fwd_loop_k(const float* __restrict__ 
 // Host dispatch.
 
 template <bool LN, bool NTS>
-void launch_fwd_cfg(int cfg, hipStream_t s, const float* x, const float* w, const float* b, float* y, float* mean,
-                    float* rstd, int64_t rows, int h, float eps) {
+void launch_fwd_cfg(int cfg, bool odd, hipStream_t s, const float* x, const float* w, const float* b, float* y,
+                    float* mean, float* rstd, int64_t rows, int h, float eps) {
+#define OXI_FWD_GO(TPR, NV, NT, KIND, NTS_)                                                                \
+  norm_fwd_k<TPR, NV, LN, NTS_, KIND, NT><<<dim3((unsigned)ceil_div(rows, NT / TPR)), dim3(NT), 0, s>>>(    \
+      x, w, b, y, mean, rstd, rows, h, eps)
 #define OXI_FWD_NT(TPR, NV, NT)                                                                            \
-  if (h == 4 * TPR * NV)                                                                                   \
-    norm_fwd_k<TPR, NV, LN, NTS, true, NT><<<dim3((unsigned)ceil_div(rows, NT / TPR)), dim3(NT), 0, s>>>(   \
-        x, w, b, y, mean, rstd, rows, h, eps);                                                             \
-  else                                                                                                     \
-    norm_fwd_k<TPR, NV, LN, NTS, false, NT><<<dim3((unsigned)ceil_div(rows, NT / TPR)), dim3(NT), 0, s>>>(  \
-        x, w, b, y, mean, rstd, rows, h, eps);
+  if (odd) OXI_FWD_GO(TPR, NV, NT, ROW_ODD, false);                                                        \
+  else if (h == 4 * TPR * NV) OXI_FWD_GO(TPR, NV, NT, ROW_FULL, NTS);                                      \
+  else OXI_FWD_GO(TPR, NV, NT, ROW_VEC, NTS);
 #define OXI_FWD(TPR, NV)                                                                                   \
   case TPR * 10 + NV:                                                                                      \
     OXI_FWD_NT(TPR, NV, row_block_threads(TPR))                                                            \
@@ -172,25 +183,35 @@ void launch_fwd_cfg(int cfg, hipStream_t s, const float* x, const float* w, cons
     OXI_FWD(256, 4)
     OXI_FWD(512, 2)
     OXI_FWD(256, 8)
+    OXI_FWD(1024, 4)
     default:
       norm_fwd_loop_k<LN><<<dim3((unsigned)rows), dim3(BS), 0, s>>>(x, w, b, y, mean, rstd, rows, h, eps);
   }
 #undef OXI_FWD
 #undef OXI_FWD1
 #undef OXI_FWD_NT
+#undef OXI_FWD_GO
 }
 
 template <bool LN>
 int launch_fwd(const float* x, const float* w, const float* b, float* y, float* mean, float* rstd,
                int64_t rows, int64_t H, float eps) {
   hipStream_t s = stream();
-  int cfg = vec_ok(H, {x, w, b, y}) ? pick_row_cfg(H / 4) : 0;
+  // rows that are no multiple of 4 floats, or not at 16-byte addresses, go
+  // through the same kernels with float4s at float alignment: layer norm of
+  // (8192, 1003) 13.4 us against 26.2 a float a thread, of (16384, 2047) 41
+  // against 88 (6.5 TB/s)
+  const bool odd = !vec_ok(H, {x, w, b, y});
+  const int64_t h4 = ceil_div(H, 4);
+  int cfg = H < 4 ? 0 : pick_row_cfg(h4);
+  if (H >= 4 && !cfg && h4 <= 4096) cfg = 10244;  // rows of up to 16384 floats: 1024 threads of 4 float4s,
+  // layer norm of (2048, 12288) 41 us against 74 re-reading the row
 #ifdef OXI_NORM_FWD_512X2
   if (cfg == 2564) cfg = 5122;
 #endif
   const int h = (int)H;
-  if (nt_stores(rows * H * 4)) launch_fwd_cfg<LN, true>(cfg, s, x, w, b, y, mean, rstd, rows, h, eps);
-  else launch_fwd_cfg<LN, false>(cfg, s, x, w, b, y, mean, rstd, rows, h, eps);
+  if (nt_stores(rows * H * 4)) launch_fwd_cfg<LN, true>(cfg, odd, s, x, w, b, y, mean, rstd, rows, h, eps);
+  else launch_fwd_cfg<LN, false>(cfg, odd, s, x, w, b, y, mean, rstd, rows, h, eps);
   return check_launch(LN ? "layer_norm_fwd" : "rms_norm_fwd");
 }
 
@@ -326,7 +347,7 @@ int oxi_layer_norm_bwd_noalloc(const float* x, const float* w, const float* mean
     if (!rc && db && cols) rc = oxi_fill(db, cols, 0.f);
     return rc;
   }
-  const int cfg = vec_ok(cols, {x, w, g, dx}) ? pick_bwd_cfg(cols / 4) : 0;
+  const int cfg = plain_bwd_cfg(cols);
   const size_t need = bwd_part_bytes(dw || db, rows, cols, cfg);
   if (need > (size_t)OXI_NOALLOC_SCRATCH_BYTES)
     return fail(OXI_INVALID_ARGUMENT,

@@ -79,6 +79,20 @@ inline int pick_bwd_cfg(int64_t h4) {
   return 0;
 }
 
+// The configuration of the plain VJP (no folded activation, no leading sum),
+// whose rows may lie anywhere: as above by the row's slots, rows of up to
+// 16384 floats on 1024 threads of 4; 0 (the loop kernel) for rows of fewer
+// than 4 floats and longer ones. Against the loop kernel, which reads single
+// floats twice and keeps its column partials in memory, layer norm's exact VJP
+// of (8192, 1003) takes 20 us instead of 123, of (16384, 2047) 75 instead of
+// 576 (5.4 TB/s), of (2048, 12288) 64 instead of 612.
+inline int plain_bwd_cfg(int64_t H) {
+  const int64_t h4 = ceil_div(H, 4);
+  if (H < 4) return 0;
+  const int cfg = pick_bwd_cfg(h4);
+  return cfg ? cfg : h4 <= 4096 ? 10244 : 0;
+}
+
 // 1024-thread (one-wave row) blocks per CU: 2 made C5's layer_norm + silu
 // VJP 43 us against 35 us at 1 (C1's rms_norm VJP unchanged)
 #ifndef OXI_BWD_BPC1024

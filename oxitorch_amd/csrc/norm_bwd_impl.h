@@ -66,11 +66,12 @@ __device__ __forceinline__ float act_vjp(float y, float g) {
 template <bool LSUM, int ACT>
 constexpr int bwd_waves_per_eu() { return LSUM && is_softmax_act(ACT) ? 4 : 1; }
 
-// FULL: rows of exactly TPR * NV float4s (H = 4 * TPR * NV), so that H and
-// the float4 count are compile-time constants: no lane is padding, and the
-// bounds checks, padding selects and row-address multiplies fold away (the
-// per-row instruction count of C5's fused softmax VJP drops by a third).
-template <int TPR, int NV, int MODE, bool LN, bool NTS, int ACT, bool LSUM, bool FULL>
+// KIND: RowKind. ROW_FULL: H and the float4 count are compile-time constants:
+// no lane is padding, and the bounds checks, padding selects and row-address
+// multiplies fold away (the per-row instruction count of C5's fused softmax
+// VJP drops by a third). ROW_ODD (plain VJP only): a row's last slot repeats
+// up to 3 floats, which stay out of the row sums and the column partials.
+template <int TPR, int NV, int MODE, bool LN, bool NTS, int ACT, bool LSUM, int KIND>
 __global__ __launch_bounds__((bwd_threads<TPR, NV, LSUM, ACT>())) __attribute__((amdgpu_waves_per_eu(bwd_waves_per_eu<LSUM, ACT>())))
 void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
                                                  const float* __restrict__ b,
@@ -79,7 +80,10 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
                                                  float* __restrict__ dx,
                                                  float* __restrict__ part, int64_t rows, int H_arg,
                                                  float* __restrict__ lsum, int64_t T) {
-  const int H = FULL ? 4 * TPR * NV : H_arg;
+  const int H = KIND == ROW_FULL ? 4 * TPR * NV : H_arg;
+  constexpr bool ODD = KIND == ROW_ODD;
+  static_assert(!ODD || (ACT == ACT_NONE && !LSUM), "odd rows: the plain VJP");
+  static_assert(TPR < 1024 || ACT == ACT_NONE, "rows of 1024 threads: the plain VJP");
   static_assert(!LSUM || TPR == 64, "the leading-sum walk takes one-wave rows");
   constexpr int NT = bwd_threads<TPR, NV, LSUM, ACT>();
   constexpr int GPB = NT / TPR;
@@ -93,7 +97,7 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
   float* comb = SPLIT ? dyn_lds : comb_static;
   const int t = threadIdx.x % TPR;
   const int gi = threadIdx.x / TPR;
-  const int h4 = H >> 2;
+  const int h4 = row_slots<KIND>(H);
   const float fH = (float)H;
   const float inv_n = 1.0f / fH;
   const f4* w4 = reinterpret_cast<const f4*>(w);
@@ -108,24 +112,25 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
   // row's prefetch, and the in-order vmcnt wait for it would also wait for
   // the prefetch. Wide rows (TPR > 64) keep them in registers; one-wave rows
   // run 16 waves to a CU at up to 128 VGPRs and read them from LDS, staged
-  // once per block. Padding lanes (c >= h4) are zeroed at use.
-  constexpr bool REG_W = TPR > 64;
+  // once per block, and so do rows of 1024 threads. Padding lanes (c >= h4)
+  // are zeroed at use.
+  constexpr bool REG_W = TPR > 64 && TPR < 1024;
   constexpr int WL = REG_W ? 1 : TPR * NV;  // float4s of w (and b) in LDS
-  __shared__ f4 wl[WL], bl[WL];
+  __shared__ f4 wl[WL], bl[TPR < 1024 ? WL : 1];
   f4 wr[NV], br[NV];
   const bool need_b = ACT != ACT_NONE && LN && b;
   if constexpr (REG_W) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int cc = min(k * TPR + t, h4 - 1);
-      wr[k] = w ? w4[cc] : f4{1.f, 1.f, 1.f, 1.f};
+      wr[k] = !w ? f4{1.f, 1.f, 1.f, 1.f} : ODD ? ld_odd(w, H, cc) : w4[cc];
       br[k] = need_b ? b4[cc] : zero;
     }
   } else {
     for (int c = threadIdx.x; c < WL; c += NT) {
       const int cc = min(c, h4 - 1);
-      wl[c] = w ? w4[cc] : f4{1.f, 1.f, 1.f, 1.f};
-      bl[c] = need_b ? b4[cc] : zero;
+      wl[c] = !w ? f4{1.f, 1.f, 1.f, 1.f} : ODD ? ld_odd(w, H, cc) : w4[cc];
+      if constexpr (TPR < 1024) bl[c] = need_b ? b4[cc] : zero;
     }
     __syncthreads();
   }
@@ -155,8 +160,13 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
     // loads keep it in L2 (non-temporal ones fetched it from HBM again, +25%
     // reads at 16 rows a position)
     constexpr bool ntl = !LSUM || (is_softmax_act(ACT) && OXI_LSUM_SPLIT_NT);
-    xt.template load_clamped<ntl>(x + r * H, h4, t);
-    gt.template load_clamped<ntl>(g + r * H, h4, t);
+    if constexpr (ODD) {
+      xt.load_odd_clamped(x + r * H, H, t);
+      gt.load_odd_clamped(g + r * H, H, t);
+    } else {
+      xt.template load_clamped<ntl>(x + r * H, h4, t);
+      gt.template load_clamped<ntl>(g + r * H, h4, t);
+    }
     inv = rstd[r];
     if constexpr (LN) mu = mean[r];
   };
@@ -238,8 +248,9 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
         gt.v[k] = zero;
       }
       xt.v[k] = xh;  // xt now holds xhat
-      pdw[k] = pdw[k] + gt.v[k] * xh;
-      if constexpr (LN) pdb[k] = pdb[k] + gt.v[k];
+      const f4 gp = without_dup<KIND>(gt.v[k], H, c);
+      pdw[k] = pdw[k] + gp * xh;
+      if constexpr (LN) pdb[k] = pdb[k] + gp;
     }
     if (dx) {
       if constexpr (MODE == OXI_NORM_VJP_REF) {
@@ -248,7 +259,8 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
           gt.v[k] = (gt.v[k] * wv_at(k)) * inv;
-          s += (gt.v[k].x + gt.v[k].y) + (gt.v[k].z + gt.v[k].w);
+          const f4 q = without_dup<KIND>(gt.v[k], H, k * TPR + t);
+          s += (q.x + q.y) + (q.z + q.w);
         }
         if constexpr (LN) {
           const float corr = (-rsum1<TPR>(s, slot())) * inv_n;
@@ -261,9 +273,10 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
           gt.v[k] = gt.v[k] * wv_at(k);
-          const f4 p = gt.v[k] * xt.v[k];
+          const f4 q = without_dup<KIND>(gt.v[k], H, k * TPR + t);
+          const f4 p = q * xt.v[k];
           sb += (p.x + p.y) + (p.z + p.w);
-          sa += (gt.v[k].x + gt.v[k].y) + (gt.v[k].z + gt.v[k].w);
+          sa += (q.x + q.y) + (q.z + q.w);
         }
         float a = 0.f;
         if constexpr (LN) a = rsum1<TPR>(sa, slot()) * inv_n;
@@ -271,7 +284,8 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
 #pragma unroll
         for (int k = 0; k < NV; ++k) gt.v[k] = ((gt.v[k] - a) - xt.v[k] * bcoef) * inv;
       }
-      gt.template store<NTS>(dx + r * H, h4, t);
+      if constexpr (ODD) gt.store_odd(dx + r * H, H, h4, t);
+      else gt.template store<NTS>(dx + r * H, h4, t);
     }
   };
   RowTile<TPR, NV> xa, ga, xb, gb;
@@ -417,9 +431,11 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
         }
       }
     }
-  } else if ((int64_t)rows <= ngroups) {
-    // at most one row per group (e.g. 4096 rows of 768): nothing to prefetch
-    if (row < rows) {
+  } else if (TPR * NV > 2048 || (int64_t)rows <= ngroups) {
+    // at most one row per group (e.g. 4096 rows of 768): nothing to prefetch;
+    // rows of 1024 threads: no registers for a second row (128 VGPRs a lane)
+#pragma unroll 1
+    for (; row < rows; row += ngroups) {
       fetch(xa, ga, ia, ma, row);
       process(xa, ga, ia, ma, row);
     }
@@ -444,7 +460,17 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int c = k * TPR + t;
-      if (c < h4) {
+      if constexpr (ODD) {
+        if (c < h4) {
+          const int e0 = min(4 * c, H - 4);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (e0 + j >= 4 * c) {  // the repeated floats belong to the slot before
+              pw[e0 + j] = pdw[k][j];
+              if (LN) pb[e0 + j] = pdb[k][j];
+            }
+        }
+      } else if (c < h4) {
         reinterpret_cast<f4*>(pw)[c] = pdw[k];
         if (LN) reinterpret_cast<f4*>(pb)[c] = pdb[k];
       }
@@ -459,9 +485,11 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
       __syncthreads();
       float* dst = plane ? pb : pw;
       for (int c = threadIdx.x; c < H; c += NT) {
-        float sum = comb[c];
+        // an odd row's last H % 4 floats end its last slot
+        const int e = ODD && c >= (H & ~3) ? 4 * h4 - H + c : c;
+        float sum = comb[e];
 #pragma unroll
-        for (int q = 1; q < GPB; ++q) sum += comb[q * ROWF + c];
+        for (int q = 1; q < GPB; ++q) sum += comb[q * ROWF + e];
         dst[c] = sum;
       }
       __syncthreads();
@@ -469,7 +497,8 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
   }
 }
 
-// Backward for any H / alignment: each block loops over its rows; the block's
+// Backward for rows of fewer than 4 floats or more than the register kernels
+// take: each block loops over its rows; the block's
 // partial row lives in global memory owned by that block alone.
 template <int MODE, bool LN>
 __global__ __launch_bounds__(BS) void norm_bwd_loop_k(const float* __restrict__ x, const float* __restrict__ w,
@@ -582,26 +611,30 @@ size_t lsum_dyn_bytes() {
 }
 
 template <bool LN, int MODE, bool NTS, int ACT>
-void launch_bwd_cfg(int cfg, hipStream_t s, int64_t nblk, int nt, const float* x, const float* w, const float* b,
+void launch_bwd_cfg(int cfg, bool odd, hipStream_t s, int64_t nblk, int nt, const float* x, const float* w, const float* b,
                     const float* mean, const float* rstd, const float* g, float* dyo, float* dx, float* part,
                     int64_t rows, int h, float* lsum, int64_t T) {
+#define OXI_BWD_GO(TPR, NV, NTS_, KIND)                                                                    \
+  norm_bwd_k<TPR, NV, MODE, LN, NTS_, ACT, false, KIND><<<dim3((unsigned)nblk), dim3(nt), 0, s>>>(         \
+      x, w, b, mean, rstd, g, dyo, dx, part, rows, h, nullptr, 0)
 #define OXI_BWD(TPR, NV)                                                                                   \
   case TPR * 10 + NV:                                                                                      \
-    if (h == 4 * TPR * NV)                                                                                 \
-      norm_bwd_k<TPR, NV, MODE, LN, NTS, ACT, false, true><<<dim3((unsigned)nblk), dim3(nt), 0, s>>>(      \
-          x, w, b, mean, rstd, g, dyo, dx, part, rows, h, nullptr, 0);                                     \
-    else                                                                                                   \
-      norm_bwd_k<TPR, NV, MODE, LN, NTS, ACT, false, false><<<dim3((unsigned)nblk), dim3(nt), 0, s>>>(     \
-          x, w, b, mean, rstd, g, dyo, dx, part, rows, h, nullptr, 0);                                     \
+    if (odd) {                                                                                             \
+      if constexpr (ACT == ACT_NONE) OXI_BWD_GO(TPR, NV, false, ROW_ODD);                                  \
+    } else if (h == 4 * TPR * NV) {                                                                        \
+      OXI_BWD_GO(TPR, NV, NTS, ROW_FULL);                                                                  \
+    } else {                                                                                               \
+      OXI_BWD_GO(TPR, NV, NTS, ROW_VEC);                                                                   \
+    }                                                                                                      \
     break;
 #define OXI_BWD_LSUM(NV)                                                                                   \
   case 640 + NV:                                                                                           \
     if (h == 4 * 64 * NV)                                                                                  \
-      norm_bwd_k<64, NV, MODE, LN, NTS, ACT, true, true>                                                   \
+      norm_bwd_k<64, NV, MODE, LN, NTS, ACT, true, ROW_FULL>                                               \
           <<<dim3((unsigned)nblk), dim3(bwd_threads<64, NV, true, ACT>()), lsum_dyn_bytes<NV, ACT>(), s>>>( \
               x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T);                                    \
     else                                                                                                   \
-      norm_bwd_k<64, NV, MODE, LN, NTS, ACT, true, false>                                                  \
+      norm_bwd_k<64, NV, MODE, LN, NTS, ACT, true, ROW_VEC>                                                \
           <<<dim3((unsigned)nblk), dim3(bwd_threads<64, NV, true, ACT>()), lsum_dyn_bytes<NV, ACT>(), s>>>( \
               x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T);                                    \
     break;
@@ -626,10 +659,16 @@ void launch_bwd_cfg(int cfg, hipStream_t s, int64_t nblk, int nt, const float* x
     OXI_BWD(512, 4)
     default:
       // vectorized shapes only when fused (the entry point checks)
-      if constexpr (ACT == ACT_NONE)
+      if constexpr (ACT == ACT_NONE) {
+        switch (cfg) {
+          OXI_BWD(1024, 4)
+          default:
         norm_bwd_loop_k<MODE, LN><<<dim3((unsigned)nblk), dim3(BS), 0, s>>>(x, w, mean, rstd, g, dx, part, rows, h);
+        }
+      }
   }
 #undef OXI_BWD
+#undef OXI_BWD_GO
 #undef OXI_BWD_LSUM
 }
 
@@ -645,8 +684,10 @@ int launch_bwd(const float* x, const float* w, const float* b, const float* mean
                void* fixed = nullptr, float* lsum = nullptr, int64_t lead = 0, size_t fixed_bytes = 0) {
   hipStream_t s = stream();
   const bool need_part = dw || (LN && db);
-  const int cfg = vec_ok(H, {x, w, b, g, dyo, dx}) ? pick_bwd_cfg(H / 4) : 0;
-  if (ACT != ACT_NONE && cfg == 0) return fail(OXI_OTHER, "norm_act_bwd: internal: unvectorized fused launch");
+  const bool odd = !vec_ok(H, {x, w, b, g, dyo, dx});
+  const bool plain = ACT == ACT_NONE && !lsum;
+  const int cfg = plain ? plain_bwd_cfg(H) : odd ? 0 : pick_bwd_cfg(H / 4);
+  if (!plain && cfg == 0) return fail(OXI_OTHER, "norm_act_bwd: internal: unvectorized fused launch");
   const int tpr = cfg ? cfg / 10 : BS;
   const bool split = lsum && is_softmax_act(ACT);
   const int nt = lsum ? (split ? LSUM_SPLIT_THREADS : LSUM_THREADS) : tpr == 64 ? (cfg % 10 <= 3 ? 1024 : 512) : tpr;  // bwd_threads<>()
@@ -676,9 +717,9 @@ int launch_bwd(const float* x, const float* w, const float* b, const float* mean
   const int h = (int)H;
   const int64_t T = lsum ? rows / lead : 0;
   if (nt_stores(rows * H * 4))
-    launch_bwd_cfg<LN, MODE, true, ACT>(cfg, s, nblk, nt, x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T);
+    launch_bwd_cfg<LN, MODE, true, ACT>(cfg, odd, s, nblk, nt, x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T);
   else
-    launch_bwd_cfg<LN, MODE, false, ACT>(cfg, s, nblk, nt, x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T);
+    launch_bwd_cfg<LN, MODE, false, ACT>(cfg, odd, s, nblk, nt, x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T);
   int rc = check_launch(LN ? "layer_norm_bwd" : "rms_norm_bwd");
   if (rc != OXI_OK) return rc;
   if (need_part) {

@@ -132,9 +132,58 @@ inline int pick_row_cfg(int64_t h4) {
   return 0;
 }
 
+// How a kernel's rows lie. ROW_FULL: exactly TPR * NV float4s at 16-byte
+// addresses, the length a compile-time constant; ROW_VEC: any multiple of 4
+// floats at 16-byte addresses; ROW_ODD: 4 or more floats at any float address.
+// Slot c of a row is its floats 4c .. 4c + 3, except that an odd row's last
+// slot is its last 4 floats: the first `dup` of them repeat floats of the slot
+// before (both lanes form and write the same values) and are left out of sums.
+enum RowKind { ROW_VEC = 0, ROW_FULL = 1, ROW_ODD = 2 };
+
+template <int KIND>
+__device__ __forceinline__ int row_slots(int H) { return KIND == ROW_ODD ? (H + 3) >> 2 : H >> 2; }
+
+// Slot c of an odd row (slots past the last re-read it).
+__device__ __forceinline__ f4 ld_odd(const float* __restrict__ row, int H, int c) {
+  return *reinterpret_cast<const f4u*>(row + min(4 * c, H - 4));
+}
+
+// v with the floats that slot c repeats set to 0 (other kinds: v).
+template <int KIND>
+__device__ __forceinline__ f4 without_dup(f4 v, int H, int c) {
+  if constexpr (KIND == ROW_ODD) {
+    const int dup = 4 * c - (H - 4);  // positive in the last slot only: 0 .. 3
+    if (dup > 0) v.x = 0.f;
+    if (dup > 1) v.y = 0.f;
+    if (dup > 2) v.z = 0.f;
+  }
+  return v;
+}
+
 template <int TPR, int NV>
 struct RowTile {
   f4 v[NV];
+
+  // An odd row of h4 slots; slots past the last are 0.
+  __device__ __forceinline__ void load_odd(const float* __restrict__ row, int H, int h4, int t) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int c = k * TPR + t;
+      v[k] = c < h4 ? ld_odd(row, H, c) : f4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  __device__ __forceinline__ void load_odd_clamped(const float* __restrict__ row, int H, int t) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v[k] = ld_odd(row, H, k * TPR + t);
+  }
+  // plain stores: neighbouring rows share cache lines
+  __device__ __forceinline__ void store_odd(float* __restrict__ row, int H, int h4, int t) const {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int c = k * TPR + t;
+      if (c < h4) *reinterpret_cast<f4u*>(row + min(4 * c, H - 4)) = v[k];
+    }
+  }
 
   __device__ __forceinline__ void load(const float* __restrict__ row, int h4, int t) {
     const f4* p = reinterpret_cast<const f4*>(row);
