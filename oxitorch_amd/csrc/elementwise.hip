@@ -10,14 +10,15 @@
 //   rows    the innermost dim is contiguous or broadcast for every operand:
 //           one block walks a chunk of one row, offsets computed once per row;
 //   tiled   an input is transposed relative to the output (its unit-stride
-//           dim is not the output's innermost dim). With float4-aligned
-//           operands one wave owns a 32x32 tile and each lane a 4x4 block,
-//           read as float4 rows along the input's unit-stride dim and
-//           written as float4 columns along the output's innermost dim, so
-//           both coalesce with no LDS; otherwise 64x64 tiles go through LDS;
+//           dim is not the output's innermost dim). One wave owns a 32x32
+//           tile and each lane a 4x4 block, read as float4 rows along the
+//           input's unit-stride dim and written as float4 columns along the
+//           output's innermost dim, so both coalesce with no LDS; dims of
+//           fewer than 4 take 64x64 tiles through LDS;
 //   generic anything else: per-element index arithmetic.
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "internal.h"
 #include "ops.h"
@@ -216,9 +217,15 @@ __global__ __launch_bounds__(BS) void map_tiled_k(F f, Plan<N> p, int jd, unsign
 // columns along its innermost dim; the transpose between them is only which
 // register goes where. Each load or store instruction of a wave covers 8
 // runs of 128 contiguous bytes; no LDS, no barriers.
+// ODD: extents, strides and addresses of any number of floats (extents of 4 or
+// more): float4s at float alignment, and the last block of a dim ends with it,
+// so it may repeat elements of the block before (both write the same values).
+// silu of (16, 1023, 768) permuted to (16, 768, 1023) takes 22 us against
+// 41.6 through LDS a float at a time, the add back 24.5 against 46.1, as long
+// as the aligned (16, 1024, 768) ones.
 constexpr int RT = 32;  // tile extent per wave in both dims
 
-template <class F, int N, unsigned TM, bool NTS>
+template <class F, int N, unsigned TM, bool NTS, bool ODD>
 __global__ __launch_bounds__(BS) void map_regt_k(F f, Plan<N> p, int jd, unsigned tiles_d, unsigned tiles_j,
                                                  unsigned tiles) {
   unsigned b = blockIdx.x * (BS / 64) + (threadIdx.x >> 6);  // this wave's tile
@@ -240,9 +247,14 @@ __global__ __launch_bounds__(BS) void map_regt_k(F f, Plan<N> p, int jd, unsigne
     for (int k = 0; k <= N; ++k) off[k] += (int64_t)c * p.st[k][q];
   }
   const int lane = threadIdx.x & 63;
-  const int gj = (int)tj * RT + 4 * (lane & 7), gd = (int)td * RT + 4 * (lane >> 3);
-  // both dims are multiples of 4: a block is wholly inside or wholly outside
-  if (gj >= (int)p.shape[jd] || gd >= (int)p.shape[d]) return;
+  int gj = (int)tj * RT + 4 * (lane & 7), gd = (int)td * RT + 4 * (lane >> 3);
+  const int nj = (int)p.shape[jd], nd = (int)p.shape[d];
+  if (gj >= nj || gd >= nd) return;
+  if constexpr (ODD) {
+    gj = min(gj, nj - 4);
+    gd = min(gd, nd - 4);
+  }  // else both dims are multiples of 4: a block is wholly inside or wholly outside
+  using V = typename std::conditional<ODD, f4u, f4>::type;
   float v[N][4][4];  // [input][jd offset c][innermost offset r]
 #pragma unroll
   for (int k = 0; k < N; ++k) {
@@ -251,7 +263,9 @@ __global__ __launch_bounds__(BS) void map_regt_k(F f, Plan<N> p, int jd, unsigne
       const int64_t sd = p.st[k + 1][d];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const f4 t = ld_stream(reinterpret_cast<const f4*>(q + gj + (int64_t)(gd + r) * sd));
+        const V* a = reinterpret_cast<const V*>(q + gj + (int64_t)(gd + r) * sd);
+        // odd rows share cache lines: plain loads
+        const f4 t = ODD ? *a : ld_stream(a);
 #pragma unroll
         for (int c = 0; c < 4; ++c) v[k][c][r] = t[c];
       }
@@ -261,7 +275,7 @@ __global__ __launch_bounds__(BS) void map_regt_k(F f, Plan<N> p, int jd, unsigne
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const float* row = q + (int64_t)(gj + c) * sj;
-        const f4 t = bc ? f4{row[0], row[0], row[0], row[0]} : *reinterpret_cast<const f4*>(row + gd);
+        const f4 t = bc ? f4{row[0], row[0], row[0], row[0]} : *reinterpret_cast<const V*>(row + gd);
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[k][c][r] = t[r];
       }
@@ -277,16 +291,19 @@ __global__ __launch_bounds__(BS) void map_regt_k(F f, Plan<N> p, int jd, unsigne
       for (int k = 0; k < N; ++k) a[k] = v[k][c][r];
       o[r] = apply<F, N>(f, a);
     }
-    st_stream<NTS>(o, reinterpret_cast<f4*>(p.y + off[0] + (int64_t)(gj + c) * p.st[0][jd] + gd));
+    V* dst = reinterpret_cast<V*>(p.y + off[0] + (int64_t)(gj + c) * p.st[0][jd] + gd);
+    if constexpr (ODD) *dst = o;
+    else st_stream<NTS>(o, dst);
   }
 }
 
 template <class F, int N, unsigned TM>
-void launch_regt(F f, const Plan<N>& p, int jd, unsigned tiles_d, unsigned tiles_j, unsigned tiles, bool nts,
+void launch_regt(F f, const Plan<N>& p, int jd, unsigned tiles_d, unsigned tiles_j, unsigned tiles, bool nts, bool odd,
                  hipStream_t s) {
   const unsigned blocks = (tiles + BS / 64 - 1) / (BS / 64);
-  if (nts) map_regt_k<F, N, TM, true><<<dim3(blocks), dim3(BS), 0, s>>>(f, p, jd, tiles_d, tiles_j, tiles);
-  else map_regt_k<F, N, TM, false><<<dim3(blocks), dim3(BS), 0, s>>>(f, p, jd, tiles_d, tiles_j, tiles);
+  if (odd) map_regt_k<F, N, TM, false, true><<<dim3(blocks), dim3(BS), 0, s>>>(f, p, jd, tiles_d, tiles_j, tiles);
+  else if (nts) map_regt_k<F, N, TM, true, false><<<dim3(blocks), dim3(BS), 0, s>>>(f, p, jd, tiles_d, tiles_j, tiles);
+  else map_regt_k<F, N, TM, false, false><<<dim3(blocks), dim3(BS), 0, s>>>(f, p, jd, tiles_d, tiles_j, tiles);
 }
 
 // ---------------------------------------------------------------------------
@@ -491,16 +508,17 @@ int launch_map(F f, const char* what, float* y, const int64_t* ys, const float* 
           }
         }
         // 32-bit block decode: every dim and the block count stay below 2^31
-        for (int q = 0; q < p.ndim && vec; ++q)
-          if (p.shape[q] >= ((int64_t)1 << 31)) vec = false;
+        bool reg = p.shape[d] >= 4 && p.shape[jd] >= 4;
+        for (int q = 0; q < p.ndim; ++q)
+          if (p.shape[q] >= ((int64_t)1 << 31)) reg = false;
         const int64_t rtiles = ceil_div(p.shape[d], RT) * ceil_div(p.shape[jd], RT) * batch;
-        if (vec && rtiles < ((int64_t)1 << 31)) {
+        if (reg && rtiles < ((int64_t)1 << 31)) {
           const unsigned ntd = (unsigned)ceil_div(p.shape[d], RT), ntj = (unsigned)ceil_div(p.shape[jd], RT);
           const unsigned nt = (unsigned)rtiles;
-          if (tmask == 1u) launch_regt<F, N, 1u>(f, p, jd, ntd, ntj, nt, nts, s);
+          if (tmask == 1u) launch_regt<F, N, 1u>(f, p, jd, ntd, ntj, nt, nts, !vec, s);
           else if constexpr (N == 2) {
-            if (tmask == 2u) launch_regt<F, N, 2u>(f, p, jd, ntd, ntj, nt, nts, s);
-            else launch_regt<F, N, 3u>(f, p, jd, ntd, ntj, nt, nts, s);
+            if (tmask == 2u) launch_regt<F, N, 2u>(f, p, jd, ntd, ntj, nt, nts, !vec, s);
+            else launch_regt<F, N, 3u>(f, p, jd, ntd, ntj, nt, nts, !vec, s);
           }
         } else
           map_tiled_k<F, N><<<dim3((unsigned)blocks), dim3(BS), 0, s>>>(f, p, jd, tmask, tiles_d, tiles_j);
