@@ -9,7 +9,8 @@
 //
 // VJP without float atomics (6 launches for 16-bit keys):
 //   1. stable LSD radix sort of (key, position) by 8-bit digits, a histogram
-//      and a scatter kernel per pass; keys are the ids wrapped to [0, len),
+//      and a scatter kernel per pass (up to 4096 ids: one kernel that counts
+//      each id's place); keys are the ids wrapped to [0, len),
 //      out-of-range ids get the sentinel key `len` (never summed) and raise
 //      the guard flag; the first scatter flags every key that occurs;
 //   2. segmented reduction over the sorted positions: one wave per (tile of
@@ -404,6 +405,78 @@ __global__ __launch_bounds__(SBS) void sort_scatter_k(const int64_t* __restrict_
   }
 }
 
+// Few ids: the whole sort in one launch. An id's place is the number of ids
+// with a smaller key, or the same key and an earlier position, so nothing is
+// exchanged between blocks: every block stages all n keys in LDS and its
+// RANK_W waves count for the same 64 ids, each over its share of the keys (four
+// to a broadcast LDS read). What bounds it is those n * n comparisons, two
+// instructions each, so it takes up to RANK_MAX ids: the gather and its VJP
+// into a (50257, 768) table take 38.1 us at 1024 ids (49.5 with the radix sort's
+// four launches), 46.0 at 4096 (52.2), and took 63.6 at 8192 (56.6). The block
+// also writes the presence flags of its share of the keys' range.
+constexpr int RANK_W = 16;             // waves a block (8: 48.6 us in all at 4096 ids against 46.0)
+constexpr int RANK_E = 64;             // ids a block ranks
+constexpr int RANK_MAX = 4096;         // ids (16 KB of keys)
+constexpr int RANK_FLAGS = 1024;       // presence flags staged at a time
+
+__global__ __launch_bounds__(RANK_W * 64) void sort_rank_k(const int64_t* __restrict__ idx, int n, int64_t len,
+                                                           int* __restrict__ keys_out, int* __restrict__ vals_out,
+                                                           int* __restrict__ present, int* __restrict__ owner_count,
+                                                           int* guard) {
+  constexpr int NT = RANK_W * 64;
+  __shared__ __align__(16) int key[RANK_MAX];
+  __shared__ int part[RANK_W][RANK_E];
+  __shared__ int flag[RANK_FLAGS];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int n4 = (n + 3) & ~3;
+  bool bad = false;
+  for (int i = t; i < n4; i += NT) key[i] = i < n ? key_from(idx[i], len, bad) : 0x7fffffff;  // past the end: after all
+  if (bad && blockIdx.x == 0) atomicOr(guard, 1);
+  if (blockIdx.x == 0 && t == 0) *owner_count = 0;
+  __syncthreads();
+  const int e0 = min((int)blockIdx.x * RANK_E, n4);
+  const int i = e0 + lane;
+  const int k = i < n ? key[i] : 0;
+  int cnt = 0;
+  // keys [j0, j1): those below e0 count when <= k, those past the 64 ids when < k
+  auto count = [&](int j0, int j1, int lim) {
+#pragma unroll 4
+    for (int j = j0; j < j1; j += 4) {
+      const int4 q = *reinterpret_cast<const int4*>(key + j);
+      cnt += (q.x < lim) + (q.y < lim) + (q.z < lim) + (q.w < lim);
+    }
+  };
+  const int per = ((n4 + RANK_W - 1) / RANK_W + 3) & ~3;
+  const int a = min(w * per, n4), b = min(a + per, n4);
+  count(a, min(b, max(a, e0)), k + 1);
+  for (int j = max(a, e0); j < min(b, e0 + RANK_E); ++j) cnt += key[j] < k + (j < i ? 1 : 0);
+  count(max(a, min(b, e0 + RANK_E)), b, k);
+  part[w][lane] = cnt;
+  __syncthreads();
+  if (w == 0 && i < n) {
+    int dst = 0;
+#pragma unroll
+    for (int q = 0; q < RANK_W; ++q) dst += part[q][lane];
+    keys_out[dst] = k;
+    vals_out[dst] = i;
+  }
+  // presence flags of keys [v0, v1)
+  const int64_t share = (len + gridDim.x - 1) / gridDim.x;
+  const int64_t v0 = min<int64_t>(blockIdx.x * share, len), v1 = min<int64_t>(v0 + share, len);
+  for (int64_t f0 = v0; f0 < v1; f0 += RANK_FLAGS) {
+    const int m = (int)min<int64_t>(RANK_FLAGS, v1 - f0);
+    for (int f = t; f < m; f += NT) flag[f] = 0;
+    __syncthreads();
+    for (int j = t; j < n; j += NT) {
+      const int64_t f = (int64_t)key[j] - f0;
+      if (f >= 0 && f < m) flag[f] = 1;
+    }
+    __syncthreads();
+    for (int f = t; f < m; f += NT) present[f0 + f] = flag[f];
+    __syncthreads();
+  }
+}
+
 // ---------------------------------------------------------------------------
 // VJP, segmented reduction. The sorted positions are cut into tiles of `st`
 // (<= 64) positions; one wave owns a (tile, 64-column-vector chunk) pair and
@@ -776,8 +849,8 @@ int check_sizes(const char* what, int64_t outer, int64_t len, int64_t inner, int
 }
 
 // The id-dependent half of the VJP: the stable sort of (key, position)
-// pairs and each key's presence flag. Built on any stream; `ready` is set
-// when it was built on the side stream.
+// pairs and each key's presence flag. Built on the library stream (few ids) or
+// the side stream; only the latter takes the events.
 struct SortPlan {
   int64_t n = 0, len = 0;
   void* ws = nullptr;  // keys, pos, keys2, pos2, count table, present, owner count
@@ -788,11 +861,20 @@ struct SortPlan {
   hipEvent_t queued = nullptr;  // the library stream's position when the plan was queued
   hipEvent_t ready = nullptr;   // recorded on the side stream after the sort
   mutable int applies = 0;  // a second apply (retain_graph) re-zeroes the owner count
+  bool side = false;        // built on the side stream
   bool recorded = false;    // `ready` holds the sort's completion
   // the library stream is already ordered after the sort (an apply waited
   // for `ready`, or saw it complete): freeing the plan needs no wait
   mutable bool ordered = false;
 };
+
+// Ids up to which a plan is sorted on the library stream instead of the side
+// stream: ordering the two costs about 30 us and 35 us of host time, the sort
+// of 16384 ids 14. Plan, gather and VJP into (50257, 768), with nothing and with
+// three layer norms of the gathered rows between: 16384 ids 84 -> 69 and 126 ->
+// 129 us (the embedding-to-softmax chain of 16 x 1024 tokens 231 us either way), 32768 107 -> 97
+// and 202 -> 203, 64 64 -> 30 and 72 -> 41; 65536 ids 152 -> 141 but 342 -> 355.
+constexpr int64_t PLAN_INLINE_MAX = 32768;
 
 int build_plan(const int64_t* idx, int64_t n, int64_t len, hipStream_t s, SortPlan* p) {
   p->n = n;
@@ -817,6 +899,15 @@ int build_plan(const int64_t* idx, int64_t n, int64_t len, hipStream_t s, SortPl
   int* tab = pos2 + n;
   p->present = tab + 256 * rtiles;
   p->owner_count = p->present + len;
+  if (n <= RANK_MAX) {
+    // blocks past the ids only write presence flags
+    const unsigned nb = (unsigned)std::max(ceil_div(n, RANK_E), std::min<int64_t>(64, ceil_div(len, RANK_FLAGS)));
+    sort_rank_k<<<dim3(nb), dim3(RANK_W * 64), 0, s>>>(idx, (int)n, len, keys, pos, p->present, p->owner_count,
+                                                       guard_flag());
+    p->ka = keys;
+    p->va = pos;
+    return check_launch("index_select_bwd/sort");
+  }
   // pass p reads (ka, va) and writes (kb, vb); pass 0 reads the ids
   const int* ka = nullptr;
   const int* va = nullptr;
@@ -1010,6 +1101,16 @@ int oxi_index_select_bwd_plan(const int64_t* idx, int64_t n, int64_t len, void**
   if (n > 0 && !idx) return fail(OXI_INVALID_ARGUMENT, "index_select_bwd_plan: NULL ids");
   OXI_CHECK_INIT();
   SortPlan* p = new SortPlan();
+  if (n <= PLAN_INLINE_MAX) {  // in order on the library stream: nothing to wait for
+    const int rc = build_plan(idx, n, len, stream(), p);
+    if (rc != OXI_OK) {
+      (void)oxi_index_select_bwd_plan_free(p);
+      return rc;
+    }
+    *plan = p;
+    return OXI_OK;
+  }
+  p->side = true;
   // the side stream starts after everything already queued on the library
   // stream: the ids' upload, and every earlier user of the plan's memory
   p->queued = take_event();
@@ -1066,7 +1167,7 @@ int oxi_index_select_bwd_plan_free(void* plan) {
     (void)hipStreamWaitEvent(stream(), p->ready, 0);
   // a plan whose build failed part-way has no completion event: kernels it
   // queued may still run on the side stream, so drain it (error path only)
-  if (!p->recorded && p->ws) (void)hipStreamSynchronize(side_stream());
+  if (p->side && !p->recorded && p->ws) (void)hipStreamSynchronize(side_stream());
   if (p->ws) ws_free(p->ws);
   give_event(p->queued);
   give_event(p->ready);
