@@ -66,12 +66,89 @@ __device__ __forceinline__ float act_vjp(float y, float g) {
 template <bool LSUM, int ACT>
 constexpr int bwd_waves_per_eu() { return LSUM && is_softmax_act(ACT) ? 4 : 1; }
 
+// Few rows: dw and db in the same launch, by blocks past the row blocks (block
+// cb owns 64 columns, its waves the 16 slices of col_finish_k) that read x and
+// g themselves, from L2: no column partials, no workspace, no second launch.
+// The sums are those of the two launches, bit for bit: GPB rows in order in
+// float32 (a block's combine), those by slices in float64 (col_finish_k).
+// Layer norm's VJP of (64, 768) takes 4.8 us against 6.8 in two launches, of
+// (256, 4096) 5.9 against 12.1, with a folded tanh GELU 4.9 against 8.3 and 9.6
+// against 12.8; at 512 rows of 768 7.3 against 8.1 but 11.4 against 8.8 with the
+// GELU, at 1024 11.9 against 7.9. Rows of 256 threads have 4 waves a block to
+// form a folded activation again: (32, 2048) 8.2 us either way, (64, 2048) 8.2
+// against 6.9.
+constexpr int FEW_MAX = 256;
+constexpr int FEW_MAX_ACT256 = 16;
+
+template <int GPB, bool LN, int ACT>
+__device__ __forceinline__ void few_columns(int cb, const float* __restrict__ x, const float* __restrict__ w,
+                                            const float* __restrict__ b, const float* __restrict__ mean,
+                                            const float* __restrict__ rstd, const float* __restrict__ g,
+                                            float* __restrict__ dw, float* __restrict__ db, int rows, int H, int waves) {
+  constexpr int FS = 16, U = GPB > 1 ? GPB : 8;  // slices; rows in flight
+  __shared__ double sw[FS][64], sb[LN ? FS : 1][64];
+  const int lane = threadIdx.x & 63;
+  const int c = cb * 64 + lane, cc = min(c, H - 1);
+  const int nb = (rows + GPB - 1) / GPB;
+  const float wc = ACT != ACT_NONE && w ? w[cc] : 1.f, bc = ACT != ACT_NONE && LN && b ? b[cc] : 0.f;
+  for (int s = threadIdx.x >> 6; s < FS; s += waves) {
+    double aw = 0.0, ab = 0.0;
+    // partial rows s, s + 16, ...: U / GPB of them at a time
+    for (int p0 = s; p0 < nb; p0 += FS * (U / GPB)) {
+      float xv[U], gv[U], iv[U], mv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int r = min((p0 + FS * (u / GPB)) * GPB + u % GPB, rows - 1);  // in range: loads issue together
+        xv[u] = x[(int64_t)r * H + cc];
+        gv[u] = g[(int64_t)r * H + cc];
+        iv[u] = rstd[r];
+        mv[u] = LN ? mean[r] : 0.f;
+      }
+      float pw = 0.f, pb = 0.f;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = u % GPB, p = p0 + FS * (u / GPB);
+        const float xh = LN ? (xv[u] - mv[u]) * iv[u] : xv[u] * iv[u];
+        float dy = gv[u];
+        if constexpr (ACT != ACT_NONE) {
+          float yv = xh;
+          if (w) yv = yv * wc;
+          if (LN && b) yv = yv + bc;
+          dy = act_vjp<ACT>(yv, dy);
+        }
+        const bool in = p * GPB + q < rows && p < nb;
+        const float tw = in ? 0.f + dy * xh : 0.f, tb = in ? 0.f + dy : 0.f;
+        pw = q == 0 ? tw : pw + tw;
+        pb = q == 0 ? tb : pb + tb;
+        if (q == GPB - 1 && p < nb) {
+          aw += (double)pw;
+          ab += (double)pb;
+        }
+      }
+    }
+    sw[s][lane] = aw;
+    if constexpr (LN) sb[s][lane] = ab;
+  }
+  __syncthreads();
+  auto total = [&](double (*v)[64]) {
+    double t = v[0][lane] + v[1][lane];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) t += v[2 * i][lane] + v[2 * i + 1][lane];
+    return (float)t;
+  };
+  if (threadIdx.x < 64 && c < H) {
+    if (dw) dw[c] = total(sw);
+    if constexpr (LN)
+      if (db) db[c] = total(sb);
+  }
+}
+
 // KIND: RowKind. ROW_FULL: H and the float4 count are compile-time constants:
 // no lane is padding, and the bounds checks, padding selects and row-address
 // multiplies fold away (the per-row instruction count of C5's fused softmax
 // VJP drops by a third). ROW_ODD (plain VJP only): a row's last slot repeats
 // up to 3 floats, which stay out of the row sums and the column partials.
-template <int TPR, int NV, int MODE, bool LN, bool NTS, int ACT, bool LSUM, int KIND>
+template <int TPR, int NV, int MODE, bool LN, bool NTS, int ACT, bool LSUM, int KIND, bool FEW = false>
 __global__ __launch_bounds__((bwd_threads<TPR, NV, LSUM, ACT>())) __attribute__((amdgpu_waves_per_eu(bwd_waves_per_eu<LSUM, ACT>())))
 void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
                                                  const float* __restrict__ b,
@@ -79,7 +156,8 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
                                                  const float* __restrict__ g, float* __restrict__ dyo,
                                                  float* __restrict__ dx,
                                                  float* __restrict__ part, int64_t rows, int H_arg,
-                                                 float* __restrict__ lsum, int64_t T) {
+                                                 float* __restrict__ lsum, int64_t T, float* __restrict__ dw,
+                                                 float* __restrict__ db, int row_blocks) {
   const int H = KIND == ROW_FULL ? 4 * TPR * NV : H_arg;
   constexpr bool ODD = KIND == ROW_ODD;
   static_assert(!ODD || (ACT == ACT_NONE && !LSUM), "odd rows: the plain VJP");
@@ -89,6 +167,13 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
   constexpr int GPB = NT / TPR;
   constexpr int ROWF = TPR * NV * 4;  // floats a group covers
   constexpr bool SPLIT = LSUM && is_softmax_act(ACT);
+  if constexpr (FEW) {
+    static_assert(!LSUM && !is_softmax_act(ACT), "few rows: the plain and elementwise-activation VJPs");
+    if ((int)blockIdx.x >= row_blocks) {  // dw, db
+      few_columns<GPB, LN, ACT>((int)blockIdx.x - row_blocks, x, w, b, mean, rstd, g, dw, db, (int)rows, H, NT / 64);
+      return;
+    }
+  }
   __shared__ float lds[2 * (NT / 64)];
   // the softmax positional-sum split combines its groups in the dynamic LDS
   // (lsum_dyn_bytes), which first stages each position's dx rows
@@ -290,6 +375,13 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
   };
   RowTile<TPR, NV> xa, ga, xb, gb;
   float ia = 0.f, ma = 0.f, ib = 0.f, mb = 0.f;
+  if constexpr (FEW) {  // one row a group
+    if (row < rows) {
+      fetch(xa, ga, ia, ma, row);
+      process(xa, ga, ia, ma, row);
+    }
+    return;
+  }
   // The scheduling barriers keep the current row's first use below the next
   // row's loads, so its wait leaves those loads in flight.
   if constexpr (LSUM && is_softmax_act(ACT)) {
@@ -613,13 +705,27 @@ size_t lsum_dyn_bytes() {
 template <bool LN, int MODE, bool NTS, int ACT>
 void launch_bwd_cfg(int cfg, bool odd, hipStream_t s, int64_t nblk, int nt, const float* x, const float* w, const float* b,
                     const float* mean, const float* rstd, const float* g, float* dyo, float* dx, float* part,
-                    int64_t rows, int h, float* lsum, int64_t T) {
+                    int64_t rows, int h, float* lsum, int64_t T, float* few_dw, float* few_db, int64_t few_blocks) {
 #define OXI_BWD_GO(TPR, NV, NTS_, KIND)                                                                    \
   norm_bwd_k<TPR, NV, MODE, LN, NTS_, ACT, false, KIND><<<dim3((unsigned)nblk), dim3(nt), 0, s>>>(         \
-      x, w, b, mean, rstd, g, dyo, dx, part, rows, h, nullptr, 0)
+      x, w, b, mean, rstd, g, dyo, dx, part, rows, h, nullptr, 0, nullptr, nullptr, 0)
+#define OXI_BWD_FEW(TPR, NV, KIND)                                                                         \
+  norm_bwd_k<TPR, NV, MODE, LN, true, ACT, false, KIND, true>                                              \
+      <<<dim3((unsigned)(nblk + few_blocks)), dim3(nt), 0, s>>>(x, w, b, mean, rstd, g, dyo, dx, nullptr,  \
+                                                                rows, h, nullptr, 0, few_dw, few_db, (int)nblk)
 #define OXI_BWD(TPR, NV)                                                                                   \
   case TPR * 10 + NV:                                                                                      \
-    if (odd) {                                                                                             \
+    if (few_blocks) {                                                                                      \
+      if constexpr (NTS && !is_softmax_act(ACT)) {                                                         \
+        if (odd) {                                                                                         \
+          if constexpr (ACT == ACT_NONE) OXI_BWD_FEW(TPR, NV, ROW_ODD);                                    \
+        } else if (h == 4 * TPR * NV) {                                                                    \
+          OXI_BWD_FEW(TPR, NV, ROW_FULL);                                                                  \
+        } else {                                                                                           \
+          OXI_BWD_FEW(TPR, NV, ROW_VEC);                                                                   \
+        }                                                                                                  \
+      }                                                                                                    \
+    } else if (odd) {                                                                                      \
       if constexpr (ACT == ACT_NONE) OXI_BWD_GO(TPR, NV, false, ROW_ODD);                                  \
     } else if (h == 4 * TPR * NV) {                                                                        \
       OXI_BWD_GO(TPR, NV, NTS, ROW_FULL);                                                                  \
@@ -632,11 +738,11 @@ void launch_bwd_cfg(int cfg, bool odd, hipStream_t s, int64_t nblk, int nt, cons
     if (h == 4 * 64 * NV)                                                                                  \
       norm_bwd_k<64, NV, MODE, LN, NTS, ACT, true, ROW_FULL>                                               \
           <<<dim3((unsigned)nblk), dim3(bwd_threads<64, NV, true, ACT>()), lsum_dyn_bytes<NV, ACT>(), s>>>( \
-              x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T);                                    \
+              x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T, nullptr, nullptr, 0);                                    \
     else                                                                                                   \
       norm_bwd_k<64, NV, MODE, LN, NTS, ACT, true, ROW_VEC>                                                \
           <<<dim3((unsigned)nblk), dim3(bwd_threads<64, NV, true, ACT>()), lsum_dyn_bytes<NV, ACT>(), s>>>( \
-              x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T);                                    \
+              x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T, nullptr, nullptr, 0);                                    \
     break;
   if (lsum) {  // one-wave rows only (lsum_check)
     switch (cfg) {
@@ -669,6 +775,7 @@ void launch_bwd_cfg(int cfg, bool odd, hipStream_t s, int64_t nblk, int nt, cons
   }
 #undef OXI_BWD
 #undef OXI_BWD_GO
+#undef OXI_BWD_FEW
 #undef OXI_BWD_LSUM
 }
 
@@ -683,7 +790,7 @@ int launch_bwd(const float* x, const float* w, const float* b, const float* mean
                const float* g, float* dyo, float* dx, float* dw, float* db, int64_t rows, int64_t H,
                void* fixed = nullptr, float* lsum = nullptr, int64_t lead = 0, size_t fixed_bytes = 0) {
   hipStream_t s = stream();
-  const bool need_part = dw || (LN && db);
+  bool need_part = dw || (LN && db);
   const bool odd = !vec_ok(H, {x, w, b, g, dyo, dx});
   const bool plain = ACT == ACT_NONE && !lsum;
   const int cfg = plain ? plain_bwd_cfg(H) : odd ? 0 : pick_bwd_cfg(H / 4);
@@ -705,6 +812,11 @@ int launch_bwd(const float* x, const float* w, const float* b, const float* mean
   if (need_part && nblk > cap) nblk = cap;
   if (!need_part && nblk > (int64_t)cu_count() * 16) nblk = (int64_t)cu_count() * 16;
   if (nblk < 1) nblk = 1;
+  // few rows, one to a group: blocks past the row blocks sum the columns
+  const bool few = need_part && !lsum && !is_softmax_act(ACT) && cfg && rows <= (ACT != ACT_NONE && tpr == 256 ? FEW_MAX_ACT256 : FEW_MAX) && rows <= nblk * gpb &&
+                   nt_stores(rows * H * 4);
+  const int64_t few_blocks = few ? ceil_div(H, 64) : 0;
+  if (few) need_part = false;
   const size_t part_bytes = need_part ? sizeof(float) * 2 * (size_t)nblk * (size_t)H : 0;
   if (fixed && part_bytes > fixed_bytes)
     return fail(OXI_OTHER, "norm VJP: internal: column partials of %zu bytes exceed the fixed buffer of %zu bytes",
@@ -717,9 +829,11 @@ int launch_bwd(const float* x, const float* w, const float* b, const float* mean
   const int h = (int)H;
   const int64_t T = lsum ? rows / lead : 0;
   if (nt_stores(rows * H * 4))
-    launch_bwd_cfg<LN, MODE, true, ACT>(cfg, odd, s, nblk, nt, x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T);
+    launch_bwd_cfg<LN, MODE, true, ACT>(cfg, odd, s, nblk, nt, x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T,
+                                         few ? dw : nullptr, few ? db : nullptr, few_blocks);
   else
-    launch_bwd_cfg<LN, MODE, false, ACT>(cfg, odd, s, nblk, nt, x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T);
+    launch_bwd_cfg<LN, MODE, false, ACT>(cfg, odd, s, nblk, nt, x, w, b, mean, rstd, g, dyo, dx, part, rows, h, lsum, T,
+                                         few ? dw : nullptr, few ? db : nullptr, few_blocks);
   int rc = check_launch(LN ? "layer_norm_bwd" : "rms_norm_bwd");
   if (rc != OXI_OK) return rc;
   if (need_part) {
