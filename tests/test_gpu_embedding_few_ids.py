@@ -51,3 +51,18 @@ def test_sequential_order_and_guard(hip, n):
         hip.sync()
     np.testing.assert_array_equal(got.numpy(), want)
     hip.sync()
+
+
+@pytest.mark.parametrize("n", [65537, 524289, 2_100_000])
+@pytest.mark.parametrize("V,hot", [(255, 0.3), (256, 1.0), (70000, 0.3)])
+def test_passes_and_tiles(hip, n, V, hot):
+    """Sorts of one, two and three passes, each counting for the next, over
+    tiles of 2048 and 8192 ids and over more tiles than a block scans itself."""
+    print("embedding passes", n, V, hot, flush=True)
+    r = np.random.default_rng(n + V)
+    ids = r.integers(0, V, n)
+    ids[r.random(n) < hot] = V - 1
+    g = r.integers(-3, 4, (n, 1)).astype(np.float32)
+    want = np.bincount(ids, g[:, 0], V)[:, None]
+    got = hip.index_select_bwd(hip.DeviceArray.from_numpy(g), (V, 1), 0, hip.DeviceArray.from_numpy(ids.astype(np.int64)))
+    np.testing.assert_array_equal(got.numpy(), want)
