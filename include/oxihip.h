@@ -357,11 +357,11 @@ int oxi_index_select(const float* src, int64_t outer, int64_t len, int64_t inner
 int oxi_index_select_bwd(const float* g, int64_t outer, int64_t len, int64_t inner,
                          const int64_t* idx, int64_t n, float* grad_src);
 /* The same VJP in two halves, so the id-dependent half leaves the backward:
- * _plan sorts the ids (a stable sort by id with each id's presence flag) on
- * the library's second stream, after everything already queued on the library
- * stream, as soon as the ids are known (at forward time); _apply makes the
- * library stream wait for the plan and runs the segment sums of g for any
- * (outer, inner) of the same ids. A plan may be applied more than once.
+ * _plan sorts the ids (a stable sort by id with each id's presence flag) as
+ * soon as they are known (at forward time): up to 32768 of them in order on the
+ * library stream, more on the library's second stream, after everything already
+ * queued on the library stream; _apply makes the library stream wait for such a
+ * plan and runs the segment sums of g for any (outer, inner) of the same ids. A plan may be applied more than once.
  * _plan_free releases it (after the library stream has passed its sort).
  * Together they compute exactly what oxi_index_select_bwd computes. The
  * plan/apply split has no counterpart in the reference (its VJP is one call,

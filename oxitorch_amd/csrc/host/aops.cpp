@@ -275,9 +275,9 @@ Var narrow(const Var& x, int64_t dim, int64_t lo, int64_t hi, int64_t by) {
 
 // ---- index_select (ops.rs:498-517, 741-769) -----------------------------------------
 
-// The VJP's id sort is queued at forward time on the library's second stream
-// (oxi_index_select_bwd_plan), where it overlaps the rest of the forward; the
-// backward only waits for it and runs the segment sums.
+// The VJP's id sort is queued at forward time (oxi_index_select_bwd_plan):
+// few ids in order, many on the library's second stream, where it overlaps the
+// rest of the forward; the backward only waits for it and runs the segment sums.
 Var index_select(const Var& x, int64_t dim, const std::vector<int64_t>& indices) {
   if (!is_grad_enabled() || !x.requires_grad()) return Var::leaf(t_index_select(x.value(), dim, indices), false);
   if (x.value().ndim() == 0) err_invalid("dim " + std::to_string(dim) + " out of range for 0-D tensor");
