@@ -11,9 +11,10 @@
 //     launch;
 //   strided (any other stride): for sum/mean/norm every output is the
 //     reference's own sequential f32 fold over its strip, so the result is
-//     bit-identical to it. Many outputs: a thread walks the strip of one or
-//     four adjacent outputs. Few outputs: a block stages the strips of 16
-//     adjacent outputs through LDS and one lane per output folds them.
+//     bit-identical to it. Many outputs, or few positions: a thread walks the
+//     strip of one or four adjacent outputs. Few outputs: a block stages the
+//     strips of 16 adjacent outputs through LDS and one lane per output folds
+//     them. reduce_route() chooses.
 // max/min fold with fmaxf/fminf (NaN ignored, as f32::max/min); argmax/argmin
 // keep the first strict winner starting from index 0, so a NaN at index 0
 // sticks and later NaNs are ignored. Indices are written as floats.
@@ -21,6 +22,7 @@
 #include <type_traits>
 
 #include "internal.h"
+#include "reduce_route.h"
 #include "rowtile.h"
 
 namespace oxi {
@@ -28,39 +30,6 @@ namespace {
 
 constexpr int BS = 256;
 constexpr int MAXD = OXI_MAX_DIMS;
-
-// Where the launch shapes change, with times on MI355X (before: one wave per
-// contiguous strip reading single floats, one thread per output or four).
-// Contiguous strips of up to WAVE_MAX_LEN floats take a wave each (mean over
-// (16384, 768) 16.3 -> 8.9 us), longer ones a block of 256 threads, or 1024
-// while there are under two strips per CU: argmax over (4096, 50257) 438 ->
-// 128 us, sum over (64, 16384) 31.6 -> 4.3 us.
-constexpr int64_t WAVE_MAX_LEN = 2048;
-// From SPLIT_MIN_LEN on, and with fewer strips than CUs, the strips are cut
-// into parts of a multiple of SPLIT_MIN_PART floats (four float4s a thread),
-// about SPLIT_BLOCKS_PER_CU a CU in all: the norm of 12.6M values 46000 ->
-// 12.9 us (3.9 TB/s), 1M values 1560 -> 7.1 us. The second launch costs about
-// 3 us, what one block takes for 30000 floats more.
-constexpr int64_t SPLIT_MIN_LEN = 65536;
-constexpr int64_t SPLIT_BLOCKS_PER_CU = 4;
-constexpr int64_t SPLIT_MIN_PART = 4096;
-// Strided strips of COLS_MIN_LEN positions or more, of up to COLS_MAX_OUT
-// outputs, go through LDS: the column sums of (16384, 768) 758 -> 59 us, of
-// (1024, 16384) 68 -> 25 us, of (4096, 8000) 298 -> 42 us, the maxima of
-// (16384, 768) 760 -> 38 us. With more outputs a thread per output fills the
-// chip: (512, 65536) 42 us there against 57 us through LDS. Two and four
-// stages of loads in flight instead of one: 61-90 us at (16384, 768), the
-// staging then holding up the fold.
-constexpr int64_t COLS_MIN_LEN = 64;
-constexpr int64_t COLS_MAX_OUT = 16384;
-
-struct RPlan {
-  int nd;              // dims other than the reduced one
-  int64_t size[MAXD];  // row-major order of the remaining dims
-  int64_t st[MAXD];
-  int64_t len;         // reduced dim size
-  int64_t rst;         // reduced dim stride
-};
 
 __device__ __forceinline__ int64_t base_of(const RPlan& p, int64_t e) {
   int64_t off = 0;
@@ -124,10 +93,6 @@ __global__ __launch_bounds__(BS) void reduce_strided_k(const float* __restrict__
     out[e] = a.result(p.len);
   }
 }
-
-constexpr bool is_arg(int k) { return k == OXI_REDUCE_ARGMAX || k == OXI_REDUCE_ARGMIN; }
-// kinds whose result depends on the order of the fold
-constexpr bool is_fold(int k) { return k == OXI_REDUCE_SUM || k == OXI_REDUCE_MEAN || k == OXI_REDUCE_NORM; }
 
 // The state of one lane or group over part of a strip. For
 // argmax/argmin it is the first winner among non-NaN values; a NaN at
@@ -193,9 +158,8 @@ __device__ __forceinline__ float strip_result(const float* s, const Part<K>& a, 
 // for 16384 positions, of the 59 us the 768 columns of such a strip take); max, min and arg* take
 // four lanes per output, each a quarter of every stage. VEC: rows of float4s
 // (columns a multiple of 4, aligned); else single floats.
-constexpr int COLS_LT = 512;   // loading threads
-constexpr int COLS_NT = COLS_LT + 64;
-constexpr int COLS_C = 16;     // outputs per block
+constexpr int COLS_NT = COLS_THREADS;
+constexpr int COLS_LT = COLS_NT - 64;  // loading threads
 constexpr int COLS_R = 512;    // positions a stage
 constexpr int COLS_LD = COLS_R + 4;  // floats between outputs in LDS: 16 lanes reading float4s touch 64 distinct banks
 constexpr int COLS_F = 32;     // positions a lane has read from LDS ahead of its fold
@@ -421,52 +385,36 @@ bool capturing(hipStream_t s) {
 template <int K>
 int launch(const float* x, const RPlan& p, int64_t nout, float* out) {
   hipStream_t s = stream();
-  if (p.rst == 1 && p.len >= 32) {
-    if (nout < cu_count() && p.len >= SPLIT_MIN_LEN && !capturing(s)) {
-      const int64_t want = ceil_div(SPLIT_BLOCKS_PER_CU * (int64_t)cu_count(), nout);
-      int64_t part = ceil_div(ceil_div(p.len, want), SPLIT_MIN_PART) * SPLIT_MIN_PART;
-      const int64_t parts = ceil_div(p.len, part);
-      Workspace ws(sizeof(Part<K>) * (size_t)(nout * parts));
-      if (ws.p) {  // else: the one-launch route below
-        reduce_parts_k<K><<<dim3((unsigned)(nout * parts)), dim3(BS), 0, s>>>(x, p, part, (int)parts, ws.as<Part<K>>());
+  ReduceRoute r = reduce_route(K, p, nout, x, out, cu_count(), true);
+  if (r.kernel == ReduceKernel::Parts) {
+    if (!capturing(s)) {
+      Workspace ws(sizeof(Part<K>) * (size_t)r.blocks);
+      if (ws.p) {
+        reduce_parts_k<K><<<dim3((unsigned)r.blocks), dim3(BS), 0, s>>>(x, p, r.part, (int)r.parts, ws.as<Part<K>>());
         if (int rc = check_launch("reduce")) return rc;
-        strip_finish_k<K><<<dim3((unsigned)nout), dim3(64), 0, s>>>(x, p, (int)parts, ws.as<Part<K>>(), out);
+        strip_finish_k<K><<<dim3((unsigned)nout), dim3(64), 0, s>>>(x, p, (int)r.parts, ws.as<Part<K>>(), out);
         return check_launch("reduce_finish");
       }
     }
-    const int tps = p.len <= WAVE_MAX_LEN ? 64 : nout < 2 * cu_count() ? 1024 : 256;
-    const int64_t blocks = tps == 64 ? ceil_div(nout * 64, BS) : nout;
-    if (blocks < ((int64_t)1 << 31)) {
-      const dim3 g((unsigned)blocks);
-      if (tps == 64) reduce_contig_k<K, 64><<<g, dim3(BS), 0, s>>>(x, p, nout, out);
-      else if (tps == 256) reduce_contig_k<K, 256><<<g, dim3(256), 0, s>>>(x, p, nout, out);
+    r = reduce_route(K, p, nout, x, out, cu_count(), false);
+  }
+  const dim3 g((unsigned)r.blocks);
+  switch (r.kernel) {
+    case ReduceKernel::Strips:
+      if (r.threads == 64) reduce_contig_k<K, 64><<<g, dim3(BS), 0, s>>>(x, p, nout, out);
+      else if (r.threads == 256) reduce_contig_k<K, 256><<<g, dim3(256), 0, s>>>(x, p, nout, out);
       else reduce_contig_k<K, 1024><<<g, dim3(1024), 0, s>>>(x, p, nout, out);
-      return check_launch("reduce");
-    }
+      break;
+    case ReduceKernel::Cols:
+      if (r.vec) reduce_cols_k<K, true><<<g, dim3(COLS_NT), 0, s>>>(x, p, r.inner, r.groups, out);
+      else reduce_cols_k<K, false><<<g, dim3(COLS_NT), 0, s>>>(x, p, r.inner, r.groups, out);
+      break;
+    case ReduceKernel::Vec:
+      if constexpr (!is_arg(K)) reduce_strided_vec_k<K><<<g, dim3(BS), 0, s>>>(x, p, nout / 4, out);
+      break;
+    default:
+      reduce_strided_k<K><<<g, dim3(BS), 0, s>>>(x, p, nout, out);
   }
-  const bool unit = p.nd > 0 && p.st[p.nd - 1] == 1;  // outputs adjacent in memory
-  // vector path: every row start 16-byte aligned
-  bool vec = unit && p.size[p.nd - 1] % 4 == 0 && p.rst % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
-  for (int d = 0; d + 1 < p.nd && vec; ++d)
-    if (p.st[d] % 4) vec = false;
-  if (unit && p.len >= COLS_MIN_LEN && nout <= COLS_MAX_OUT) {
-    const int64_t inner = p.size[p.nd - 1];
-    const int64_t groups = ceil_div(inner, COLS_C);
-    const dim3 g((unsigned)(nout / inner * groups));
-    if (vec) reduce_cols_k<K, true><<<g, dim3(COLS_NT), 0, s>>>(x, p, inner, groups, out);
-    else reduce_cols_k<K, false><<<g, dim3(COLS_NT), 0, s>>>(x, p, inner, groups, out);
-    return check_launch("reduce");
-  }
-  if constexpr (!is_arg(K)) {
-    if (vec && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
-      const int64_t nout4 = nout / 4;
-      const int64_t blocks = std::min<int64_t>(ceil_div(nout4, BS), (int64_t)cu_count() * 64);
-      reduce_strided_vec_k<K><<<dim3((unsigned)std::max<int64_t>(blocks, 1)), dim3(BS), 0, s>>>(x, p, nout4, out);
-      return check_launch("reduce");
-    }
-  }
-  const int64_t blocks = std::min<int64_t>(ceil_div(nout, BS), (int64_t)cu_count() * 64);
-  reduce_strided_k<K><<<dim3((unsigned)std::max<int64_t>(blocks, 1)), dim3(BS), 0, s>>>(x, p, nout, out);
   return check_launch("reduce");
 }
 
@@ -509,6 +457,7 @@ int oxi_reduce(int kind, const float* x, const int64_t* xs, const int64_t* shape
   if (!out || (!x && p.len)) return fail(OXI_INVALID_ARGUMENT, "reduce: NULL tensor pointer");
   OXI_CHECK_INIT();
   if (p.len == 0) return oxi_fill(out, nout, 0.f);
+  simplify(p);
   switch (kind) {
     case OXI_REDUCE_SUM: return launch<OXI_REDUCE_SUM>(x, p, nout, out);
     case OXI_REDUCE_MEAN: return launch<OXI_REDUCE_MEAN>(x, p, nout, out);

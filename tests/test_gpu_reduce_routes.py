@@ -65,6 +65,26 @@ def test_strided_strips_keep_the_sequential_order(hip, shape, dim):
                                       err_msg=kind)
 
 
+# full: the extents the view is cut from (its strides), rows of 1 to 4 outputs
+@pytest.mark.parametrize("shape,full,dim", [((70, 100, 1), (70, 100, 1), 0), ((70, 100, 1), (70, 101, 3), 1),
+                                            ((65, 64, 4), (65, 64, 4), 0), ((9, 65, 2), (9, 65, 2), 1),
+                                            ((3000, 64, 3), (3000, 64, 3), 1), ((3000, 64, 4), (3001, 64, 8), 1),
+                                            ((2, 600, 1, 3), (2, 600, 5, 3), 1), ((700, 1, 1), (700, 2, 2), 0)])
+def test_narrow_rows_of_outputs(hip, shape, full, dim):
+    """Outputs that do not lie side by side, dims of size 1 and dims that
+    merge: the sequential fold's bits by either strided kernel."""
+    print("reduce narrow", shape, full, dim, flush=True)
+    from oracle import ref
+
+    whole = np.random.default_rng(sum(full)).standard_normal(full, dtype=np.float32)
+    x = whole[tuple(slice(0, n) for n in shape)]
+    buf = hip.DeviceArray.from_numpy(whole)
+    strides = hip.row_major_strides(full)
+    for kind in KINDS:
+        np.testing.assert_array_equal(_run(hip, kind, buf, shape, strides, dim, 0),
+                                      ref.reduce(kind, np.ascontiguousarray(x), dim), err_msg=kind)
+
+
 @pytest.mark.parametrize("rows,cols,dim", [(4, 70000, 1), (4, 700, 1), (700, 20, 0)])
 def test_first_winner_and_nan_rules(hip, rows, cols, dim):
     """Ties go to the first position, a NaN counts only at position 0, strips
