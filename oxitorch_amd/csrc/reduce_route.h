@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cstdint>
 
+#include "launch_limits.h"
 #include "oxihip.h"
 
 namespace oxi {
@@ -85,7 +86,7 @@ enum class ReduceKernel { Parts, Strips, Cols, Vec, Threads };
 
 struct ReduceRoute {
   ReduceKernel kernel;
-  int threads;            // of a block
+  int threads;            // of a block (Strips: of a strip; 64: four to a block)
   int64_t blocks;
   int64_t part, parts;    // Parts: positions in a part, parts in a strip
   int64_t inner, groups;  // Cols: adjacent outputs in a row, blocks in a row
@@ -110,9 +111,9 @@ inline ReduceRoute reduce_route(int kind, const RPlan& p, int64_t nout, const fl
       return r;
     }
     r.kernel = ReduceKernel::Strips;
-    r.threads = p.len <= WAVE_MAX_LEN ? 64 : nout < 2 * cus ? 1024 : 256;
-    r.blocks = r.threads == 64 ? ceil(nout * 64, 256) : nout;
-    if (r.blocks < ((int64_t)1 << 31)) return r;
+    r.threads = p.len <= WAVE_MAX_LEN || !grid_fits(nout, 256) ? 64 : nout < 2 * cus ? 1024 : 256;
+    r.blocks = r.threads == 64 ? ceil(nout, 256 / 64) : nout;
+    if (grid_fits(r.blocks, std::max(r.threads, 256))) return r;
   }
   const bool unit = p.nd > 0 && p.st[p.nd - 1] == 1;  // outputs adjacent in memory
   r.inner = unit ? p.size[p.nd - 1] : 1;

@@ -147,3 +147,14 @@ def test_captured_long_strip(hip):
         if exe.value:
             rt.hipGraphExecDestroy(exe)
         rt.hipGraphDestroy(graph)
+
+
+def test_more_long_strips_than_a_grid_of_blocks_holds(hip):
+    """2^24 and a few strips of one broadcast row: 256 threads each would be a
+    grid of more than 2^32 threads."""
+    n, length = 2 ** 24 + 5, 2051
+    print("reduce many strips", n, length, flush=True)
+    x = np.random.default_rng(1).integers(-8, 9, length).astype(np.float32)  # sums are exact in any order
+    buf = hip.DeviceArray.from_numpy(x)
+    got = _run(hip, "sum", buf, (n, length), (0, 1), 1, 0)
+    assert (got == x.sum(dtype=np.float64)).all()

@@ -131,3 +131,18 @@ def test_columns_route_is_bounded(lib):
             if r["kernel"] == "cols":
                 assert r["blocks"] <= (16384 if kind in ("max", "min") else 16 * CUS)
                 assert r["blocks"] == rows * r["groups"] and rows * inner <= 16384
+
+
+@pytest.mark.parametrize("length", [32, 2048, 2049, 50257])
+def test_grids_stay_below_the_thread_limit(lib, length):
+    """A launch counts its threads in 32 bits: from 2^24 long strips on a wave
+    takes each, and strips that do not fit so go a thread each."""
+    for n in (2 ** 20, 2 ** 24 - 1, 2 ** 24, 2 ** 24 + 1, 2 ** 26 - 4, 2 ** 26, 2 ** 33):
+        r = route(lib, (n, length), 1)
+        block = max(r["threads"], 256)
+        assert r["blocks"] < 2 ** 31 and r["blocks"] * block < 2 ** 32, (n, r)
+        if n < 2 ** 26:
+            assert r["kernel"] == "strips" and r["threads"] == (64 if length <= 2048 or n >= 2 ** 24 else 256), (n, r)
+            assert r["blocks"] * (block // r["threads"]) >= n
+        else:
+            assert r["kernel"] == "threads"
