@@ -202,10 +202,7 @@ int launch_fwd(const float* x, const float* w, const float* b, float* y, float* 
   // (8192, 1003) 13.4 us against 26.2 a float a thread, of (16384, 2047) 41
   // against 88 (6.5 TB/s)
   const bool odd = !vec_ok(H, {x, w, b, y});
-  const int64_t h4 = ceil_div(H, 4);
-  int cfg = H < 4 ? 0 : pick_row_cfg(h4);
-  if (H >= 4 && !cfg && h4 <= 4096) cfg = 10244;  // rows of up to 16384 floats: 1024 threads of 4 float4s,
-  // layer norm of (2048, 12288) 41 us against 74 re-reading the row
+  int cfg = norm_fwd_cfg(rows, H);
 #ifdef OXI_NORM_FWD_512X2
   if (cfg == 2564) cfg = 5122;
 #endif

@@ -11,6 +11,8 @@
 
 #include <cstdint>
 
+#include "row_cfg.h"
+
 namespace oxi {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
@@ -109,28 +111,6 @@ __device__ __forceinline__ void div_by_sum(f4 (&v)[NV], float s) {
 #define OXI_NT_STORE_HI (320 << 20)
 #endif
 inline bool nt_stores(int64_t bytes) { return bytes < (int64_t)OXI_NT_STORE_LO || bytes > (int64_t)OXI_NT_STORE_HI; }
-
-// Threads per block of a row kernel whose rows take TPR threads: 256 (several
-// rows per block) when TPR divides 256, else one row per block of TPR.
-constexpr int row_block_threads(int tpr) { return (256 % tpr == 0) ? 256 : tpr; }
-
-// (TPR, NV) for rows of h4 float4s, encoded TPR*10 + NV; 0 when the row does
-// not fit in registers. Rows keep several float4s per lane: measured on
-// MI355X, one float4 per lane (192 threads per 768-float row, 1024 per
-// 4096-float row) made the layer-norm forward 30% slower, the block-wide
-// reductions over many waves costing more than the access pattern gains;
-// 512 x 2 for a 4096-float row measured the same as 256 x 4 (layer-norm
-// forward at (16384, 4096): 88.8-89.5 us against 87.7-89.3 us).
-inline int pick_row_cfg(int64_t h4) {
-  if (h4 <= 64) return 641;
-  if (h4 <= 128) return 642;
-  if (h4 <= 192) return 643;
-  if (h4 <= 256) return 644;
-  if (h4 <= 512) return 2562;
-  if (h4 <= 1024) return 2564;
-  if (h4 <= 2048) return 2568;
-  return 0;
-}
 
 // How a kernel's rows lie. ROW_FULL: exactly TPR * NV float4s at 16-byte
 // addresses, the length a compile-time constant; ROW_VEC: any multiple of 4
