@@ -20,6 +20,7 @@
 
 #include "internal.h"
 #include "rowtile.h"
+#include "softmax_mid.h"
 
 namespace oxi {
 namespace {
@@ -389,29 +390,6 @@ __global__ __launch_bounds__(NT) void sm_bwd_mid_k(const float* __restrict__ y, 
   }
 }
 
-// The launch of a middle-dim kernel: NT threads, TX units by TY positions a
-// block (TX * TY = NT), NV positions a thread (0: streamed).
-struct MidShape {
-  int nt, tx, ty, nv;
-  int64_t units, total, blocks;
-};
-
-MidShape mid_shape(int64_t outer, int64_t len, int64_t inner) {
-  MidShape m;
-  const int w = inner >= 4 ? 4 : 1;
-  const int nv = w == 4 ? 8 : 16;  // positions a thread holds at most
-  m.units = ceil_div(inner, w);
-  m.total = outer * m.units;
-  m.nt = len <= 32 * nv ? 256 : 1024;
-  m.ty = 1;
-  while ((int64_t)m.ty * nv < len && m.ty < m.nt / 8) m.ty <<= 1;
-  m.tx = m.nt / m.ty;
-  const int64_t per = ceil_div(len, m.ty);
-  m.nv = per <= nv / 4 ? nv / 4 : per <= nv ? nv : 0;
-  m.blocks = ceil_div(m.total, m.tx);
-  return m;
-}
-
 // ---------------------------------------------------------------------------
 // Cross-entropy.
 
@@ -776,8 +754,11 @@ int launch_fwd(const float* x, float* y, int64_t outer, int64_t len, int64_t inn
 #undef OXI_SMF
 #undef OXI_SMF_GO
   } else {
-    const MidShape m = mid_shape(outer, len, inner);
-    OXI_MID(sm_fwd_mid_k, x, y)
+    for (int64_t o0 = 0, oc = mid_outer_max(len, inner); o0 < outer; o0 += oc) {
+      const MidShape m = mid_shape(std::min(oc, outer - o0), len, inner);
+      const int64_t at = o0 * len * inner;
+      OXI_MID(sm_fwd_mid_k, x + at, y + at)
+    }
   }
   return check_launch(LOG ? "log_softmax_fwd" : "softmax_fwd");
 }
@@ -816,8 +797,11 @@ int launch_bwd(const float* y, const float* g, float* dx, int64_t outer, int64_t
 #undef OXI_SMB
 #undef OXI_SMB_GO
   } else {
-    const MidShape m = mid_shape(outer, len, inner);
-    OXI_MID(sm_bwd_mid_k, y, g, dx)
+    for (int64_t o0 = 0, oc = mid_outer_max(len, inner); o0 < outer; o0 += oc) {
+      const MidShape m = mid_shape(std::min(oc, outer - o0), len, inner);
+      const int64_t at = o0 * len * inner;
+      OXI_MID(sm_bwd_mid_k, y + at, g + at, dx + at)
+    }
   }
   return check_launch(LOG ? "log_softmax_bwd" : "softmax_bwd");
 }

@@ -11,8 +11,15 @@ ROOT = Path(__file__).resolve().parents[1]
 
 SRC = r"""
 #include "row_cfg.h"
+#include "softmax_mid.h"
 extern "C" int norm_fwd_cfg(int64_t rows, int64_t H) { return oxi::norm_fwd_cfg(rows, H); }
 extern "C" int block_threads(int tpr) { return oxi::row_block_threads(tpr); }
+extern "C" int64_t mid_outer_max(int64_t len, int64_t inner) { return oxi::mid_outer_max(len, inner); }
+extern "C" void mid_shape(int64_t outer, int64_t len, int64_t inner, int64_t* v) {
+  const oxi::MidShape m = oxi::mid_shape(outer, len, inner);
+  const int64_t q[] = {m.nt, m.tx, m.ty, m.nv, m.units, m.total, m.blocks};
+  for (int i = 0; i < 7; ++i) v[i] = q[i];
+}
 """
 
 
@@ -22,7 +29,15 @@ def lib(tmp_path_factory):
     (d / "limits.cpp").write_text(SRC)
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-Wall", "-Werror", f"-I{ROOT / 'include'}",
                     f"-I{ROOT / 'oxitorch_amd' / 'csrc'}", str(d / "limits.cpp"), "-o", str(d / "limits.so")], check=True)
-    return ctypes.CDLL(str(d / "limits.so"))
+    lib = ctypes.CDLL(str(d / "limits.so"))
+    lib.mid_outer_max.restype = ctypes.c_int64
+    return lib
+
+
+def mid_shape(lib, outer, length, inner):
+    v = (ctypes.c_int64 * 7)()
+    lib.mid_shape(ctypes.c_int64(outer), ctypes.c_int64(length), ctypes.c_int64(inner), v)
+    return dict(zip(("nt", "tx", "ty", "nv", "units", "total", "blocks"), v))
 
 
 @pytest.mark.parametrize("H", [3, 4, 1003, 4096, 8192, 8193, 12288, 16384, 16385])
@@ -35,3 +50,18 @@ def test_norm_forward(lib, H):
         threads = cfg // 10 if cfg else 256
         block = lib.block_threads(threads)
         assert -(-rows // (block // threads)) * block < 2 ** 32, (rows, H, cfg)
+
+
+@pytest.mark.parametrize("length", [1, 2, 16, 17, 32, 33, 128, 150, 256, 257, 512, 513, 1024, 2048, 2049, 100000])
+@pytest.mark.parametrize("inner", [2, 3, 4, 5, 4096, 10 ** 6])
+def test_middle_dim_softmax(lib, length, inner):
+    """A launch takes as many outer indices as its grid holds: 2^30 of (17, 2)
+    (146 GB) ran on a thread a column, and take several threads a column now."""
+    most = lib.mid_outer_max(ctypes.c_int64(length), ctypes.c_int64(inner))
+    for outer in (1, most, min(most, 2 ** 31)):
+        m = mid_shape(lib, outer, length, inner)
+        assert m["blocks"] < 2 ** 31 and m["blocks"] * m["nt"] < 2 ** 32, m
+        assert m["blocks"] * m["tx"] >= m["total"] == outer * m["units"] and m["tx"] * m["ty"] == m["nt"]
+    # one more outer index than that would pass the limit, or nearly (a block's worth)
+    m = mid_shape(lib, most + 2 * m["tx"] + 1, length, inner)
+    assert m["blocks"] * m["nt"] >= 2 ** 32 - 2 * m["nt"]
