@@ -706,18 +706,16 @@ int check_olen(const char* what, int64_t outer, int64_t len, int64_t inner, std:
 #define OXI_MID_GO(K, W, NV, NT, ...)                                                                       \
   K<LOG, W, NV, NT><<<dim3((unsigned)m.blocks), dim3(NT), 0, s>>>(__VA_ARGS__, len, inner, m.units, m.total,   \
                                                                  m.tx, m.ty)
-#define OXI_MID_NT(K, W, NV, ...)                                                                           \
-  if (m.nt == 256) OXI_MID_GO(K, W, NV, 256, __VA_ARGS__);                                                  \
-  else OXI_MID_GO(K, W, NV, 1024, __VA_ARGS__);
-#define OXI_MID(K, ...)                                                                                     \
-  if (inner >= 4) {                                                                                         \
-    if (m.nv == 2) { OXI_MID_NT(K, 4, 2, __VA_ARGS__) }                                                     \
-    else if (m.nv == 8) { OXI_MID_NT(K, 4, 8, __VA_ARGS__) }                                                \
-    else { OXI_MID_NT(K, 4, 0, __VA_ARGS__) }                                                               \
-  } else {                                                                                                  \
-    if (m.nv == 4) { OXI_MID_NT(K, 1, 4, __VA_ARGS__) }                                                     \
-    else if (m.nv == 16) { OXI_MID_NT(K, 1, 16, __VA_ARGS__) }                                              \
-    else { OXI_MID_NT(K, 1, 0, __VA_ARGS__) }                                                               \
+#define OXI_MID_W(K, W, FEW, MOST, ...)                                                                    \
+  if (m.nv == 0) OXI_MID_GO(K, W, 0, 1024, __VA_ARGS__); /* mid_shape: streamed on 1024 threads only, */   \
+  else if (m.nv == FEW) OXI_MID_GO(K, W, FEW, 256, __VA_ARGS__); /* few positions on 256 only */           \
+  else if (m.nt == 256) OXI_MID_GO(K, W, MOST, 256, __VA_ARGS__);                                          \
+  else OXI_MID_GO(K, W, MOST, 1024, __VA_ARGS__);
+#define OXI_MID(K, ...)                                                                                    \
+  if (inner >= 4) {                                                                                        \
+    OXI_MID_W(K, 4, 2, 8, __VA_ARGS__)                                                                     \
+  } else {                                                                                                 \
+    OXI_MID_W(K, 1, 4, 16, __VA_ARGS__)                                                                    \
   }
 
 template <bool LOG>

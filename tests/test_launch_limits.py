@@ -65,3 +65,10 @@ def test_middle_dim_softmax(lib, length, inner):
     # one more outer index than that would pass the limit, or nearly (a block's worth)
     m = mid_shape(lib, most + 2 * m["tx"] + 1, length, inner)
     assert m["blocks"] * m["nt"] >= 2 ** 32 - 2 * m["nt"]
+
+
+def test_middle_dim_softmax_kernels(lib):
+    """The shapes whose kernels exist: streamed on 1024 threads, few positions on 256."""
+    for inner, few, most in ((2, 4, 16), (3, 4, 16), (4, 2, 8), (5, 2, 8), (1000, 2, 8)):
+        got = {(m["nv"], m["nt"]) for m in (mid_shape(lib, 1, n, inner) for n in [*range(1, 5000), 10 ** 5, 10 ** 9])}
+        assert got == {(0, 1024), (few, 256), (most, 256), (most, 1024)}
