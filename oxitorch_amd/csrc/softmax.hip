@@ -395,6 +395,7 @@ __global__ __launch_bounds__(NT) void sm_bwd_mid_k(const float* __restrict__ y, 
 
 constexpr int CE_BS = 256;
 constexpr int CE_U = 4;   // forward: float4 loads in flight per thread per step
+constexpr int CE_SHORT = 320;  // forward: odd rows of up to this many classes go a float a thread
 constexpr int CE_BU = 1;  // backward: float4s per thread (one per thread streams fastest)
 
 // The reference picks the target's log-probability as
@@ -416,10 +417,14 @@ __device__ __forceinline__ f4 drop_lane(const f4& v, int j) {
 // it with CE_U float4s in flight a thread, at whatever float alignment the row
 // has, and the last C % 4 logits on their own. HBM bounds it: 4096 rows of
 // 50257 classes take 136-160 us (5.1-6.0 TB/s) where single floats took 330.
+// SHORT: rows of up to CE_SHORT classes, a float a thread: most threads have
+// no float4 of theirs, and the others' chains and the tail are what the block
+// waits for (rows of 33 classes at (127100, 33) 137 us against 171 as float4s,
+// of 301 at (55738, 301) 77 against 80; of 385 at (43577, 385) 63.5 against 62.6).
 // lse[row] = max + log(sum exp(x - max));
 // picked[row] = (x[t] - max) - log(sum)  (the reference's ls[row, t]), or
 // NaN where the reference's one-hot product makes it NaN (onehot_nan).
-template <int NT>
+template <int NT, bool SHORT>
 __global__ __launch_bounds__(NT) void ce_fwd_k(const float* __restrict__ logits, const int64_t* __restrict__ targets,
                                                float* __restrict__ lse, float* __restrict__ picked, int64_t n, int C,
                                                int* __restrict__ guard) {
@@ -431,44 +436,52 @@ __global__ __launch_bounds__(NT) void ce_fwd_k(const float* __restrict__ logits,
   if (bad) tg = 0;
   float mn = -NEG_INF;
   Online o;
-  const f4u* p = reinterpret_cast<const f4u*>(xr);
-  const int c4 = C >> 2;
-  const int ct = (int)(tg >> 2);
-  const int jt = (int)(tg & 3);
-  int c = threadIdx.x;
-  for (; c + (CE_U - 1) * NT < c4; c += CE_U * NT) {
-    f4 v[CE_U];
-#pragma unroll
-    for (int u = 0; u < CE_U; ++u) v[u] = ld_stream(p + c + u * NT);
-#pragma unroll
-    for (int u = 0; u < CE_U; ++u) mn = fminf(mn, min4(c + u * NT == ct ? drop_lane(v[u], jt) : v[u]));
-    float cm = max4(v[0]);
-#pragma unroll
-    for (int u = 1; u < CE_U; ++u) cm = fmaxf(cm, max4(v[u]));
-    if (cm > o.m) {
-      o.s = (o.m == NEG_INF) ? 0.f : o.s * expf(o.m - cm);
-      o.m = cm;
+  if constexpr (SHORT) {
+    for (int c = threadIdx.x; c < C; c += NT) {
+      const float v = xr[c];
+      o.add1(v);
+      if (c != tg) mn = fminf(mn, v);
     }
-    if (o.m != NEG_INF) {
-      float acc = 0.f;
+  } else {
+    const f4u* p = reinterpret_cast<const f4u*>(xr);
+    const int c4 = C >> 2;
+    const int ct = (int)(tg >> 2);
+    const int jt = (int)(tg & 3);
+    int c = threadIdx.x;
+    for (; c + (CE_U - 1) * NT < c4; c += CE_U * NT) {
+      f4 v[CE_U];
 #pragma unroll
-      for (int u = 0; u < CE_U; ++u) acc += sum4(exp4(v[u] - o.m));
-      o.s += acc;
-    } else {
+      for (int u = 0; u < CE_U; ++u) v[u] = ld_stream(p + c + u * NT);
 #pragma unroll
-      for (int u = 0; u < CE_U; ++u) o.add4(v[u]);
+      for (int u = 0; u < CE_U; ++u) mn = fminf(mn, min4(c + u * NT == ct ? drop_lane(v[u], jt) : v[u]));
+      float cm = max4(v[0]);
+#pragma unroll
+      for (int u = 1; u < CE_U; ++u) cm = fmaxf(cm, max4(v[u]));
+      if (cm > o.m) {
+        o.s = (o.m == NEG_INF) ? 0.f : o.s * expf(o.m - cm);
+        o.m = cm;
+      }
+      if (o.m != NEG_INF) {
+        float acc = 0.f;
+#pragma unroll
+        for (int u = 0; u < CE_U; ++u) acc += sum4(exp4(v[u] - o.m));
+        o.s += acc;
+      } else {
+#pragma unroll
+        for (int u = 0; u < CE_U; ++u) o.add4(v[u]);
+      }
     }
-  }
-  for (; c < c4; c += NT) {
-    const f4 v = p[c];
-    o.add4(v);
-    mn = fminf(mn, min4(c == ct ? drop_lane(v, jt) : v));
-  }
-  if ((int)threadIdx.x < (C & 3)) {
-    const int e = 4 * c4 + threadIdx.x;
-    const float v = xr[e];
-    o.add1(v);
-    if (e != tg) mn = fminf(mn, v);
+    for (; c < c4; c += NT) {
+      const f4 v = p[c];
+      o.add4(v);
+      mn = fminf(mn, min4(c == ct ? drop_lane(v, jt) : v));
+    }
+    if ((int)threadIdx.x < (C & 3)) {
+      const int e = 4 * c4 + threadIdx.x;
+      const float v = xr[e];
+      o.add1(v);
+      if (e != tg) mn = fminf(mn, v);
+    }
   }
   group_online<NT>(o, lds);
   mn = -group_max<NT>(-mn, lds);
@@ -649,6 +662,16 @@ __global__ __launch_bounds__(CE_BS) void ce_bwd_k(const float* __restrict__ logi
         }
         st_stream<NTS>(e * scale, q + c);
       }
+    }
+  } else if (C <= CE_BS) {
+    // short odd rows: a float a thread, in one block (a float4 a thread leaves
+    // three quarters of it idle: (127100, 33) 59 us against 67, (65793, 255) 34
+    // against 45, but (65280, 257), two blocks a row, 58 against 42)
+    const int c = threadIdx.x;
+    if (c < C) {
+      float e = exp_le0(xr[c] - l);
+      if (c == t) e -= 1.f;
+      dr[c] = e * scale;
     }
   } else {
     // Rows at any float alignment: the gradient's 16-byte granules, whole in
@@ -908,10 +931,12 @@ int ce_forward(const char* what, const float* logits, const int64_t* targets, fl
 #undef OXI_CE_GO
     default:
       // fewer rows than two a CU: 1024 threads to a long row
-      if (n < 2 * cu_count() && c > 16384)
-        ce_fwd_k<1024><<<grid, dim3(1024), 0, stream()>>>(logits, targets, lse, pk, n, (int)c, guard_flag());
+      if (c <= CE_SHORT)
+        ce_fwd_k<CE_BS, true><<<grid, dim3(CE_BS), 0, stream()>>>(logits, targets, lse, pk, n, (int)c, guard_flag());
+      else if (n < 2 * cu_count() && c > 16384)
+        ce_fwd_k<1024, false><<<grid, dim3(1024), 0, stream()>>>(logits, targets, lse, pk, n, (int)c, guard_flag());
       else
-        ce_fwd_k<CE_BS><<<grid, dim3(CE_BS), 0, stream()>>>(logits, targets, lse, pk, n, (int)c, guard_flag());
+        ce_fwd_k<CE_BS, false><<<grid, dim3(CE_BS), 0, stream()>>>(logits, targets, lse, pk, n, (int)c, guard_flag());
   }
   if (int rc = check_launch(what)) return rc;
   ce_mean_k<<<1, 1024, 0, stream()>>>(picked.as<float>(), n, loss);

@@ -60,6 +60,14 @@ def test_cross_entropy(hip, n, c, xs, ds):
     assert (np.abs(_rows_back(db, (n, c), ds) - d / n) <= bound).all()
 
 
+@pytest.mark.parametrize("n,c", [(70, 33), (7, 255), (7, 256), (7, 257), (5, 319), (5, 320), (5, 321), (70000, 6)])
+@pytest.mark.parametrize("xs,ds", [(0, 0), (1, 3)])
+def test_cross_entropy_short_rows(hip, n, c, xs, ds):
+    """Both sides of the lengths where a row goes from a float a thread to
+    float4s, in the forward (320) and in the gradient (256)."""
+    test_cross_entropy(hip, n, c, xs, ds)
+
+
 @pytest.mark.parametrize("layer,mode", [(True, "exact"), (True, "ref"), (False, "exact"), (False, "ref")])
 @pytest.mark.parametrize("rows,H,skip", [(5, 1, 0), (5, 3, 1), (3, 4, 1), (70, 5, 0), (600, 7, 3), (20, 255, 2), (700, 513, 0),
                                          (17, 769, 1), (300, 1023, 0), (40, 1026, 2), (3, 2050, 0), (300, 4097, 1),
