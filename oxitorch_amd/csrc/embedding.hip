@@ -7,10 +7,11 @@
 // with float4 accesses, the rows' loads issued together; threads per block
 // are the row's float4 count rounded up to whole waves.
 //
-// VJP without float atomics (5 launches for 16-bit keys):
+// VJP without float atomics (6 launches for 16-bit keys, 5 or 3 of few ids):
 //   1. stable LSD radix sort of (key, position) by 8-bit digits, a histogram
-//      and then a scatter kernel per pass (up to 4096 ids: one kernel that counts
-//      each id's place); keys are the ids wrapped to [0, len),
+//      and a scatter kernel per pass (of few ids the scatters count for the
+//      next pass; up to 4096 ids take one kernel that counts each id's place);
+//      keys are the ids wrapped to [0, len),
 //      out-of-range ids get the sentinel key `len` (never summed) and raise
 //      the guard flag; the first scatter flags every key that occurs;
 //   2. segmented reduction over the sorted positions: one wave per (tile of
@@ -196,20 +197,17 @@ __global__ __launch_bounds__(BS) void batch_gather_k(BatchArgs a, int64_t len, c
 // Keys are the ids wrapped to [0, len); an out-of-range id gets the sentinel
 // key `len` (sorted last, never summed) and raises the guard flag. A block owns
 // a tile of SBS * IPT consecutive elements. Per pass:
-//   sort_hist_k    the first pass's per-tile digit counts (LDS integer
-//                  atomics: exact) into a tile-major table
-//                  cnt[tile * 256 + digit];
+//   sort_hist_k    per-tile digit counts (LDS integer atomics: exact) into a
+//                  tile-major table cnt[tile * 256 + digit];
 //   sort_scatter_k each block first derives its tile's 256 output offsets
 //                  from the whole table (digit-major exclusive prefix: the
 //                  stable order), then sends each element to its digit's
 //                  offset plus the number of earlier elements of the tile with
 //                  that digit (wave ballots + per-wave LDS counts).
-//                  It also adds the element to the next pass's table, by
-//                  integer atomics in memory (exact whatever their order),
-//                  so the later passes need no histogram launch of about
-//                  4 us: plan, gather and VJP into (50257, 768) 68.6 -> 67.4
-//                  us at 16384 ids, 159.2 -> 156.7 at 65536, with 200000 keys
-//                  (three passes, rows of 64 floats) 95.5 -> 93.8.
+//                  Of few ids (sort_chained) it also adds the element to the
+//                  next pass's table, by integer atomics in memory (exact
+//                  whatever their order), so that the later passes need no
+//                  histogram launch of about 4 us.
 // Tables of more than 256 tiles are scanned once by sort_offsets_k instead.
 // The first pass reads the int64 ids directly and flags every key present.
 
@@ -266,30 +264,42 @@ __device__ __forceinline__ void column_sums(const int* __restrict__ tab, int nti
   }
 }
 
-// The first pass's counts. Also clears the later passes' tables (nnext ints),
-// this call's present-key flags and its owner count.
-template <int IPT>
-__global__ __launch_bounds__(SBS) void sort_hist_k(const int64_t* __restrict__ idx, int64_t n, int64_t len,
-                                                   int* __restrict__ tab, int* __restrict__ next, int64_t nnext,
-                                                   int* __restrict__ present, int* __restrict__ owner_count,
-                                                   int* guard) {
+// A pass's counts. The first pass reads the ids and also clears the later
+// passes' tables (nnext ints), this call's present-key flags and its owner count.
+template <int IPT, bool FROM_IDX>
+__global__ __launch_bounds__(SBS) void sort_hist_k(const int64_t* __restrict__ idx, const int* __restrict__ keys,
+                                                   int64_t n, int64_t len, int shift, int* __restrict__ tab,
+                                                   int* __restrict__ next, int64_t nnext, int* __restrict__ present,
+                                                   int* __restrict__ owner_count, int* guard) {
   __shared__ int cnt[256];
   const int t = threadIdx.x;
   cnt[t] = 0;
   __syncthreads();
   const int64_t base = (int64_t)blockIdx.x * (SBS * IPT);
-  int64_t raw[IPT];
+  int k[IPT];
+  if constexpr (FROM_IDX) {
+    int64_t raw[IPT];
 #pragma unroll
-  for (int i = 0; i < IPT; ++i) raw[i] = idx[min<int64_t>(base + i * SBS + t, n - 1)];
-  bool bad = false;
+    for (int i = 0; i < IPT; ++i) raw[i] = idx[min<int64_t>(base + i * SBS + t, n - 1)];
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < IPT; ++i) k[i] = (base + i * SBS + t < n) ? key_from(raw[i], len, bad) : -1;
+    if (bad) atomicOr(guard, 1);
+  } else {
+#pragma unroll
+    for (int i = 0; i < IPT; ++i) k[i] = keys[min<int64_t>(base + i * SBS + t, n - 1)];
+#pragma unroll
+    for (int i = 0; i < IPT; ++i)
+      if (base + i * SBS + t >= n) k[i] = -1;
+  }
 #pragma unroll
   for (int i = 0; i < IPT; ++i)
-    if (base + i * SBS + t < n)
-      atomicAdd(&cnt[key_from(raw[i], len, bad) & 255], 1);  // LDS integer atomics: exact counts
-  if (bad) atomicOr(guard, 1);
-  for (int64_t v = (int64_t)blockIdx.x * SBS + t; v < nnext; v += (int64_t)gridDim.x * SBS) next[v] = 0;
-  for (int64_t v = (int64_t)blockIdx.x * SBS + t; v < len; v += (int64_t)gridDim.x * SBS) present[v] = 0;
-  if (blockIdx.x == 0 && t == 0) *owner_count = 0;
+    if (k[i] >= 0) atomicAdd(&cnt[(k[i] >> shift) & 255], 1);  // LDS integer atomics: exact counts
+  if constexpr (FROM_IDX) {
+    for (int64_t v = (int64_t)blockIdx.x * SBS + t; v < nnext; v += (int64_t)gridDim.x * SBS) next[v] = 0;
+    for (int64_t v = (int64_t)blockIdx.x * SBS + t; v < len; v += (int64_t)gridDim.x * SBS) present[v] = 0;
+    if (blockIdx.x == 0 && t == 0) *owner_count = 0;
+  }
   __syncthreads();
   tab[(int64_t)blockIdx.x * 256 + t] = cnt[t];
 }
@@ -322,7 +332,8 @@ __device__ __forceinline__ unsigned long long same_digit(unsigned long long amon
 // How a scatter block finds its 256 output offsets.
 enum { OFFS_TABLE = 0, OFFS_SCAN_COUNTS = 1 };
 
-template <int IPT, bool FROM_IDX, int OFFS>
+// NEXT: also count for the next pass.
+template <int IPT, bool FROM_IDX, int OFFS, bool NEXT>
 __global__ __launch_bounds__(SBS) void sort_scatter_k(const int64_t* __restrict__ idx, const int* __restrict__ keys,
                                                       const int* __restrict__ vals, int64_t n, int64_t len, int shift,
                                                       int ntiles, const int* __restrict__ tab, int* __restrict__ next,
@@ -382,7 +393,7 @@ __global__ __launch_bounds__(SBS) void sort_scatter_k(const int64_t* __restrict_
     const int64_t p = tile0 + r * SBS + t;
     const bool valid = p < n;
     const int k = kk[r], v = vv[r];
-    int dtile = 0;  // the output tile
+    [[maybe_unused]] int dtile = 0;  // the output tile
     const int d = (k >> shift) & 255;
     const unsigned long long peers = same_digit(__ballot(valid), d);
 #pragma unroll
@@ -402,7 +413,7 @@ __global__ __launch_bounds__(SBS) void sort_scatter_k(const int64_t* __restrict_
       }
       dtile = dst / (SBS * IPT);
     }
-    if (next) {
+    if constexpr (NEXT) {
       // the next pass's counts: one add for a wave's elements of one next
       // digit and this digit, as far as they go to one tile (their places are
       // adjacent), so that hot keys add once a wave
@@ -832,27 +843,47 @@ __global__ __launch_bounds__(256) void seg_fixup_k(int64_t outer, int64_t inner,
   }
 }
 
-// Pass ps of `passes`; tab holds a count table of `ntiles` tiles for each.
+// Whether the scatters count for the next pass. The counting is an atomic an
+// element, where the histogram launch that it saves costs 4 us whatever the
+// ids, so it pays for few ids, and only while they spread over the counters
+// (n <= 16 len). The whole VJP of rows of 4 floats, with launches of their own
+// -> counted by the scatters, us: 16384 ids of 50257 36.7 -> 33.2, of 5000 28.5
+// -> 25.1, of 300 33.0 -> 33.2 (90% of them one id 37.5 -> 38.5); 32768 of
+// 50257 36.4 -> 34.0, of 1000 41.5 -> 42.3; 65536 of 50257 51.8 -> 51.4, of 300
+// 42.1 -> 43.3; 131072 of 50257 62.8 -> 64.3, of 5000 50.9 -> 59.0; 2M of 50257
+// 318 -> 375.
+constexpr int64_t SORT_CHAIN_MAX = 32768;
+bool sort_chained(int64_t n, int64_t len) { return n <= SORT_CHAIN_MAX && n <= 16 * len; }
+
+// Pass ps of `passes` with the count table `tab`; chained: the next pass's
+// table follows it, and this one's is there already unless ps is 0.
 template <int IPT>
-void sort_pass(hipStream_t s, int ps, int passes, int64_t n, int64_t len, int ntiles, const int64_t* idx, const int* ka,
-               const int* va, int* kb, int* vb, int* tab, int* present, int* owner_count) {
+void sort_pass(hipStream_t s, int ps, int passes, bool chained, int64_t n, int64_t len, int ntiles, const int64_t* idx,
+               const int* ka, const int* va, int* kb, int* vb, int* tab, int* present, int* owner_count) {
   const int shift = 8 * ps;
   const unsigned nb = (unsigned)ntiles;
   int* gd = guard_flag();
   const bool self = ntiles <= SELF_SCAN_MAX;
   const int64_t table = (int64_t)ntiles * 256;
-  int* next = ps + 1 < passes ? tab + table : nullptr;
+  int* next = chained && ps + 1 < passes ? tab + table : nullptr;
   if (ps == 0)
-    sort_hist_k<IPT><<<nb, SBS, 0, s>>>(idx, n, len, tab, next, table * (passes - 1), present, owner_count, gd);
+    sort_hist_k<IPT, true><<<nb, SBS, 0, s>>>(idx, nullptr, n, len, shift, tab, next, next ? table * (passes - 1) : 0,
+                                              present, owner_count, gd);
+  else if (!chained)
+    sort_hist_k<IPT, false><<<nb, SBS, 0, s>>>(nullptr, ka, n, len, shift, tab, nullptr, 0, nullptr, nullptr, gd);
   if (!self) sort_offsets_k<<<1, SBS, 0, s>>>(tab, ntiles);
-#define OXI_SCATTER(FROM_IDX, OFFS, ...) \
-  sort_scatter_k<IPT, FROM_IDX, OFFS><<<nb, SBS, 0, s>>>(__VA_ARGS__, n, len, shift, ntiles, tab, next, kb, vb, present, gd)
+#define OXI_SCATTER(FROM_IDX, OFFS, NEXT, ...)                                                                   \
+  sort_scatter_k<IPT, FROM_IDX, OFFS, NEXT><<<nb, SBS, 0, s>>>(__VA_ARGS__, n, len, shift, ntiles, tab, next, kb, vb, \
+                                                               present, gd)
+  constexpr bool FEW = IPT == 2;  // the tiles of SORT_CHAIN_MAX ids
   if (ps == 0) {
-    if (self) OXI_SCATTER(true, OFFS_SCAN_COUNTS, idx, nullptr, nullptr);
-    else OXI_SCATTER(true, OFFS_TABLE, idx, nullptr, nullptr);
+    if (FEW && next) OXI_SCATTER(true, OFFS_SCAN_COUNTS, FEW, idx, nullptr, nullptr);
+    else if (self) OXI_SCATTER(true, OFFS_SCAN_COUNTS, false, idx, nullptr, nullptr);
+    else OXI_SCATTER(true, OFFS_TABLE, false, idx, nullptr, nullptr);
   } else {
-    if (self) OXI_SCATTER(false, OFFS_SCAN_COUNTS, nullptr, ka, va);
-    else OXI_SCATTER(false, OFFS_TABLE, nullptr, ka, va);
+    if (FEW && next) OXI_SCATTER(false, OFFS_SCAN_COUNTS, FEW, nullptr, ka, va);
+    else if (self) OXI_SCATTER(false, OFFS_SCAN_COUNTS, false, nullptr, ka, va);
+    else OXI_SCATTER(false, OFFS_TABLE, false, nullptr, ka, va);
   }
 #undef OXI_SCATTER
 }
@@ -877,7 +908,7 @@ int check_sizes(const char* what, int64_t outer, int64_t len, int64_t inner, int
 // the side stream; only the latter takes the events.
 struct SortPlan {
   int64_t n = 0, len = 0;
-  void* ws = nullptr;  // keys, pos, keys2, pos2, a count table a pass, present, owner count
+  void* ws = nullptr;  // keys, pos, keys2, pos2, count table (one a pass: sort_chained), present, owner count
   const int* ka = nullptr;  // sorted keys and their positions
   const int* va = nullptr;
   int* present = nullptr;
@@ -913,7 +944,9 @@ int build_plan(const int64_t* idx, int64_t n, int64_t len, hipStream_t s, SortPl
   int passes = 0;
   for (int64_t m = len; m > 0; m >>= 8) ++passes;  // keys are in [0, len]
   if (passes == 0) passes = 1;
-  const size_t ints = 4 * (size_t)n + 256 * (size_t)rtiles * (size_t)passes + (size_t)len + 1;
+  const bool chained = sort_chained(n, len);
+  const int64_t tables = chained ? passes : 1;
+  const size_t ints = 4 * (size_t)n + 256 * (size_t)rtiles * (size_t)tables + (size_t)len + 1;
   p->ws = ws_alloc(ints * sizeof(int));
   if (!p->ws) return fail_alloc("index_select_bwd: sort workspace");
   int* keys = static_cast<int*>(p->ws);
@@ -921,7 +954,7 @@ int build_plan(const int64_t* idx, int64_t n, int64_t len, hipStream_t s, SortPl
   int* keys2 = pos + n;
   int* pos2 = keys2 + n;
   int* tab = pos2 + n;
-  p->present = tab + 256 * rtiles * passes;
+  p->present = tab + 256 * rtiles * tables;
   p->owner_count = p->present + len;
   if (n <= RANK_MAX) {
     // blocks past the ids only write presence flags
@@ -940,10 +973,10 @@ int build_plan(const int64_t* idx, int64_t n, int64_t len, hipStream_t s, SortPl
   for (int ps = 0; ps < passes; ++ps) {
     int* kb = bufk[ps & 1];
     int* vb = bufv[ps & 1];
-    int* pt = tab + ps * 256 * rtiles;
-    if (ipt == 2) sort_pass<2>(s, ps, passes, n, len, (int)rtiles, idx, ka, va, kb, vb, pt, p->present, p->owner_count);
-    else if (ipt == 8) sort_pass<8>(s, ps, passes, n, len, (int)rtiles, idx, ka, va, kb, vb, pt, p->present, p->owner_count);
-    else sort_pass<32>(s, ps, passes, n, len, (int)rtiles, idx, ka, va, kb, vb, pt, p->present, p->owner_count);
+    int* pt = chained ? tab + ps * 256 * rtiles : tab;
+    if (ipt == 2) sort_pass<2>(s, ps, passes, chained, n, len, (int)rtiles, idx, ka, va, kb, vb, pt, p->present, p->owner_count);
+    else if (ipt == 8) sort_pass<8>(s, ps, passes, chained, n, len, (int)rtiles, idx, ka, va, kb, vb, pt, p->present, p->owner_count);
+    else sort_pass<32>(s, ps, passes, chained, n, len, (int)rtiles, idx, ka, va, kb, vb, pt, p->present, p->owner_count);
     ka = kb;
     va = vb;
   }

@@ -27,6 +27,13 @@ def test_exact_sums(hip, n, V, D, hot):
     plan.free()
 
 
+@pytest.mark.parametrize("n,V", [(4800, 300), (4801, 300), (32768, 2048), (32768, 2047), (32768, 70000), (32769, 70000)])
+def test_passes_counted_by_the_scatter_or_on_their_own(hip, n, V):
+    """Both sides of the sizes where a pass's counts come from the scatter
+    before it (two and three passes)."""
+    test_exact_sums(hip, n, V, 3, 0.3)
+
+
 @pytest.mark.parametrize("n", [5, 4096])
 def test_sequential_order_and_guard(hip, n):
     """Short runs add their rows in position order; an id out of range is
