@@ -327,8 +327,9 @@ __device__ __forceinline__ Part<K> strip_part(const float* __restrict__ s, int64
   return a[0];
 }
 
-// A strip per group of TPS threads.
-template <int K, int TPS>
+// A strip per group of TPS threads. SHORT (strips of up to WAVE_SHORT_LEN): its
+// lanes read single floats.
+template <int K, int TPS, bool SHORT = false>
 __global__ __launch_bounds__((TPS > BS ? TPS : BS)) void reduce_contig_k(const float* __restrict__ x, RPlan p,
                                                                          int64_t nout, float* __restrict__ out) {
   constexpr int NT = TPS > BS ? TPS : BS;
@@ -337,7 +338,16 @@ __global__ __launch_bounds__((TPS > BS ? TPS : BS)) void reduce_contig_k(const f
   const int64_t e = (int64_t)blockIdx.x * (NT / TPS) + threadIdx.x / TPS;
   if (e >= nout) return;  // TPS > 64: one strip per block, the whole block leaves together
   const float* s = x + base_of(p, e);
-  const Part<K> a = strip_part<K, TPS>(s, 0, p.len, t, lds);
+  Part<K> a;
+  if constexpr (SHORT) {
+    static_assert(TPS == 64, "short strips: a wave each");
+    a = Part<K>::none();
+    for (int k = t; k < (int)p.len; k += TPS) a.add(s[k], k);
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) a.merge(part_xor<K>(a, m));
+  } else {
+    a = strip_part<K, TPS>(s, 0, p.len, t, lds);
+  }
   if (t == 0) out[e] = strip_result<K>(s, a, p.len);
 }
 
@@ -401,7 +411,8 @@ int launch(const float* x, const RPlan& p, int64_t nout, float* out) {
   const dim3 g((unsigned)r.blocks);
   switch (r.kernel) {
     case ReduceKernel::Strips:
-      if (r.threads == 64) reduce_contig_k<K, 64><<<g, dim3(BS), 0, s>>>(x, p, nout, out);
+      if (p.len <= WAVE_SHORT_LEN) reduce_contig_k<K, 64, true><<<g, dim3(BS), 0, s>>>(x, p, nout, out);
+      else if (r.threads == 64) reduce_contig_k<K, 64><<<g, dim3(BS), 0, s>>>(x, p, nout, out);
       else if (r.threads == 256) reduce_contig_k<K, 256><<<g, dim3(256), 0, s>>>(x, p, nout, out);
       else reduce_contig_k<K, 1024><<<g, dim3(1024), 0, s>>>(x, p, nout, out);
       break;

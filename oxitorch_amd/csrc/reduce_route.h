@@ -25,6 +25,11 @@ struct RPlan {
 // while there are under two strips per CU: argmax over (4096, 50257) 438 ->
 // 128 us, sum over (64, 16384) 31.6 -> 4.3 us.
 constexpr int64_t WAVE_MAX_LEN = 2048;
+// Those of up to WAVE_SHORT_LEN read single floats, as float4s half the lanes
+// and more would have nothing to do: sums over (524288, 32) 77 us against 98,
+// (262144, 64) 40.5 against 50, (131072, 128) 25.1 against 26.0, but (83886,
+// 200) 23.8 against 19.0.
+constexpr int64_t WAVE_SHORT_LEN = 128;
 // From SPLIT_MIN_LEN on, and with fewer strips than CUs, the strips are cut
 // into parts of a multiple of SPLIT_MIN_PART floats (four float4s a thread),
 // about SPLIT_BLOCKS_PER_CU a CU in all: the norm of 12.6M values 46000 ->
@@ -86,7 +91,7 @@ enum class ReduceKernel { Parts, Strips, Cols, Vec, Threads };
 
 struct ReduceRoute {
   ReduceKernel kernel;
-  int threads;            // of a block (Strips: of a strip; 64: four to a block)
+  int threads;            // of a block (Strips: of a strip; 64: four strips to a block of 256)
   int64_t blocks;
   int64_t part, parts;    // Parts: positions in a part, parts in a strip
   int64_t inner, groups;  // Cols: adjacent outputs in a row, blocks in a row

@@ -65,6 +65,13 @@ def test_strided_strips_keep_the_sequential_order(hip, shape, dim):
                                       err_msg=kind)
 
 
+@pytest.mark.parametrize("rows,length,skip", [(5, 33, 0), (3, 63, 1), (6, 64, 0), (2, 65, 0), (9, 127, 2), (4, 128, 0),
+                                              (4, 128, 3), (4, 129, 0), (5, 131, 1)])
+def test_short_strips(hip, rows, length, skip):
+    """Both sides of the length up to which a wave's lanes read single floats."""
+    test_contiguous_strips(hip, rows, length, skip)
+
+
 # full: the extents the view is cut from (its strides), rows of 1 to 4 outputs
 @pytest.mark.parametrize("shape,full,dim", [((70, 100, 1), (70, 100, 1), 0), ((70, 100, 1), (70, 101, 3), 1),
                                             ((65, 64, 4), (65, 64, 4), 0), ((9, 65, 2), (9, 65, 2), 1),
