@@ -38,6 +38,7 @@ constexpr int64_t WAVE_SHORT_LEN = 128;
 constexpr int64_t SPLIT_MIN_LEN = 65536;
 constexpr int64_t SPLIT_BLOCKS_PER_CU = 4;
 constexpr int64_t SPLIT_MIN_PART = 4096;
+constexpr int64_t SPLIT_MAX_PARTS = 1024;  // in a strip (LDS holds their states in a captured launch)
 // Strided strips of COLS_MIN_LEN positions or more, of up to COLS_MAX_OUT
 // outputs, go through LDS: the column sums of (16384, 768) 758 -> 59 us, of
 // (1024, 16384) 68 -> 25 us, of (4096, 8000) 298 -> 42 us, the maxima of
@@ -98,16 +99,14 @@ struct ReduceRoute {
   bool vec;               // Cols: float4 rows
 };
 
-// The launch of a simplified plan. `workspace`: the launch may take one (the
-// Parts route needs it).
-inline ReduceRoute reduce_route(int kind, const RPlan& p, int64_t nout, const float* x, const float* out, int cus,
-                                bool workspace) {
+// The launch of a simplified plan.
+inline ReduceRoute reduce_route(int kind, const RPlan& p, int64_t nout, const float* x, const float* out, int cus) {
   const auto ceil = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   const auto aligned = [](const float* q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
   ReduceRoute r{};
   if (p.rst == 1 && p.len >= 32) {
-    if (nout < cus && p.len >= SPLIT_MIN_LEN && workspace) {
-      const int64_t want = ceil(SPLIT_BLOCKS_PER_CU * (int64_t)cus, nout);
+    if (nout < cus && p.len >= SPLIT_MIN_LEN) {
+      const int64_t want = std::min(ceil(SPLIT_BLOCKS_PER_CU * (int64_t)cus, nout), SPLIT_MAX_PARTS);
       r.kernel = ReduceKernel::Parts;
       r.threads = 256;
       r.part = ceil(ceil(p.len, want), SPLIT_MIN_PART) * SPLIT_MIN_PART;

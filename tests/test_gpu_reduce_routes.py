@@ -156,6 +156,61 @@ def test_captured_long_strip(hip):
         rt.hipGraphDestroy(graph)
 
 
+@pytest.mark.parametrize("rows,length", [(1, 65536), (1, 200_003), (3, 1_000_001), (250, 65_541)])
+def test_long_strips_have_the_same_bits_without_a_workspace(hip, rows, length):
+    """Under capture, and when the workspace is refused, one launch forms the
+    parts of a long strip that the eager call spreads over the chip."""
+    import ctypes
+
+    from test_gpu_graph import CAPTURE_MODE_RELAXED, _runtime
+
+    print("reduce without a workspace", rows, length, flush=True)
+    rt = _runtime()
+    x = np.random.default_rng(length).standard_normal((rows, length), dtype=np.float32)
+    x[0, length - 7] = np.nan
+    buf = hip.DeviceArray.from_numpy(x)
+    st, sh = hip._i64arr((length, 1)), hip._i64arr((rows, length))
+    outs = {k: hip.DeviceArray((rows,)) for k in KINDS}
+
+    def call(kind, o):
+        hip.call("oxi_reduce", hip.REDUCE.index(kind), buf.ptr, st, sh, 2, 1, o.ptr)
+
+    want = {k: _run(hip, k, buf, (rows, length), (length, 1), 1, 0) for k in KINDS}
+    for k in KINDS:
+        o = hip.DeviceArray.from_numpy(np.full(rows, -1, np.float32))
+        hip.lib.oxi_hip_debug_fail_alloc_after(1)
+        try:
+            call(k, o)
+        finally:
+            hip.lib.oxi_hip_debug_fail_alloc_after(0)
+        np.testing.assert_array_equal(o.numpy().view(np.uint32), want[k].view(np.uint32), err_msg=k)
+    stream, graph, exe = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    hip.check(hip.lib.oxi_hip_stream(ctypes.byref(stream)))
+    hip.sync()
+    assert rt.hipStreamBeginCapture(stream, CAPTURE_MODE_RELAXED) == 0
+    try:
+        for k in KINDS:
+            call(k, outs[k])
+    finally:
+        rc = rt.hipStreamEndCapture(stream, ctypes.byref(graph))
+    assert rc == 0 and graph.value
+    try:
+        assert rt.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0) == 0
+        for replay in range(3):
+            for k in KINDS:
+                hip.call("oxi_fill", outs[k].ptr, rows, -1.0)
+            hip.sync()
+            assert rt.hipGraphLaunch(exe, stream) == 0
+            hip.sync()
+            for k in KINDS:
+                np.testing.assert_array_equal(outs[k].numpy().view(np.uint32), want[k].view(np.uint32),
+                                              err_msg=f"{k}, replay {replay}")
+    finally:
+        if exe.value:
+            rt.hipGraphExecDestroy(exe)
+        rt.hipGraphDestroy(graph)
+
+
 def test_more_long_strips_than_a_grid_of_blocks_holds(hip):
     """2^24 and a few strips of one broadcast row: 256 threads each would be a
     grid of more than 2^32 threads."""

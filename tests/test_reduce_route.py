@@ -29,14 +29,14 @@ static RPlan plan(const int64_t* shape, const int64_t* st, int nd, int dim, int6
   simplify(p);
   return p;
 }
-// r: kernel, threads, blocks, parts, inner, groups, vec
+// r: kernel, threads, blocks, part, parts, inner, groups, vec
 extern "C" void route(const int64_t* shape, const int64_t* st, int nd, int dim, int kind, int64_t x, int cus,
-                      int workspace, int64_t* r) {
+                      int64_t* r) {
   int64_t nout;
   const RPlan p = plan(shape, st, nd, dim, &nout);
-  const ReduceRoute q = reduce_route(kind, p, nout, reinterpret_cast<const float*>(x), nullptr, cus, workspace);
-  const int64_t v[] = {(int64_t)q.kernel, q.threads, q.blocks, q.parts, q.inner, q.groups, q.vec};
-  for (int i = 0; i < 7; ++i) r[i] = v[i];
+  const ReduceRoute q = reduce_route(kind, p, nout, reinterpret_cast<const float*>(x), nullptr, cus);
+  const int64_t v[] = {(int64_t)q.kernel, q.threads, q.blocks, q.part, q.parts, q.inner, q.groups, q.vec};
+  for (int i = 0; i < 8; ++i) r[i] = v[i];
 }
 // the offset of every output's strip
 extern "C" void offsets(const int64_t* shape, const int64_t* st, int nd, int dim, int64_t* out) {
@@ -76,11 +76,10 @@ def row_major(shape):
     return st
 
 
-def route(lib, shape, dim, kind="sum", strides=None, x=0, workspace=True):
-    r = (ctypes.c_int64 * 7)()
-    lib.route(_arr(shape), _arr(strides or row_major(shape)), len(shape), dim, KINDS.index(kind), ctypes.c_int64(x), CUS,
-              int(workspace), r)
-    return dict(zip(("kernel", "threads", "blocks", "parts", "inner", "groups", "vec"), [KERNELS[r[0]], *r[1:]]))
+def route(lib, shape, dim, kind="sum", strides=None, x=0):
+    r = (ctypes.c_int64 * 8)()
+    lib.route(_arr(shape), _arr(strides or row_major(shape)), len(shape), dim, KINDS.index(kind), ctypes.c_int64(x), CUS, r)
+    return dict(zip(("kernel", "threads", "blocks", "part", "parts", "inner", "groups", "vec"), [KERNELS[r[0]], *r[1:]]))
 
 
 @pytest.mark.parametrize("shape", [(1,), (5,), (3, 1), (1, 3, 1, 4), (2, 3, 4), (4, 1, 1, 5, 2), (2, 1, 2, 1, 3, 2)])
@@ -146,3 +145,12 @@ def test_grids_stay_below_the_thread_limit(lib, length):
             assert r["blocks"] * (block // r["threads"]) >= n
         else:
             assert r["kernel"] == "threads"
+
+
+def test_parts_of_a_strip(lib):
+    """They cover it, none empty, and their states fit a block's LDS."""
+    for n, length in itertools.product((1, 2, 3, 17, 255), (65536, 65537, 1048583, 10 ** 8, 2 ** 31)):
+        r = route(lib, (n, length), 1)
+        part = r["part"]
+        assert r["kernel"] == "parts" and r["blocks"] == n * r["parts"] and r["parts"] <= 1024
+        assert part % 4096 == 0 and (r["parts"] - 1) * part < length <= r["parts"] * part
