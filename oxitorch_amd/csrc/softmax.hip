@@ -681,10 +681,9 @@ __global__ __launch_bounds__(CE_BS) void ce_bwd_k(const float* __restrict__ logi
     // 264-275 us (6.0-6.2 TB/s) where a float a thread took 550.
     const int head = min((int)((0 - (reinterpret_cast<uintptr_t>(dr) >> 2)) & 3u), C);
     const int c4 = (C - head) >> 2;
-#pragma unroll
-    for (int u = 0; u < CE_BU; ++u) {
-      const int c = blockIdx.x * (CE_BS * CE_BU) + u * CE_BS + threadIdx.x;
-      if (c >= c4) break;
+    static_assert(CE_BU == 1, "odd rows: one float4 a thread, as the grid has them");
+    const int c = blockIdx.x * CE_BS + threadIdx.x;
+    if (c < c4) {
       const int e0 = head + 4 * c;
       f4 e = exp4(ld_stream(reinterpret_cast<const f4u*>(xr + e0)) - l);
 #pragma unroll
