@@ -34,6 +34,13 @@ def test_passes_counted_by_the_scatter_or_on_their_own(hip, n, V):
     test_exact_sums(hip, n, V, 3, 0.3)
 
 
+@pytest.mark.parametrize("n", [1, 4096])
+def test_few_ids_of_many_rows(hip, n):
+    """The one-launch sort's 64 blocks write the presence flags of 46876 rows
+    each, 1024 at a time, the last block's share cut."""
+    test_exact_sums(hip, n, 3_000_001, 1, 0.3)
+
+
 @pytest.mark.parametrize("n", [5, 4096])
 def test_sequential_order_and_guard(hip, n):
     """Short runs add their rows in position order; an id out of range is

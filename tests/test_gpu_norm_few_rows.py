@@ -59,3 +59,55 @@ def test_only_one_of_dw_and_db(hip):
         for k in range(3):
             if need[k]:
                 np.testing.assert_array_equal(got[k].numpy().view(np.uint32), both[k].numpy().view(np.uint32))
+
+
+def test_captured(hip):
+    """Up to 256 rows dw and db need no workspace, so the call can be captured:
+    three replays on new inputs have the eager call's bits."""
+    import ctypes
+
+    from test_gpu_graph import CAPTURE_MODE_RELAXED, _runtime
+
+    print("norm few rows, captured", flush=True)
+    rt = _runtime()
+    rows, H = 256, 1003
+    D = hip.DeviceArray
+    x, g, dx = D((rows, H)), D((rows, H)), D((rows, H))
+    w, dw, db = D.from_numpy(np.linspace(0.5, 1.5, H, dtype=np.float32)), D((H,)), D((H,))
+    mean, rstd = D((rows,)), D((rows,))
+
+    def call():
+        hip.call("oxi_layer_norm_bwd", x.ptr, w.ptr, mean.ptr, rstd.ptr, g.ptr, dx.ptr, dw.ptr, db.ptr, rows, H,
+                 hip.NORM_VJP["exact"])
+
+    stream, graph, exe = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    hip.check(hip.lib.oxi_hip_stream(ctypes.byref(stream)))
+    hip.sync()
+    held = hip.memory_stats()[0]
+    assert rt.hipStreamBeginCapture(stream, CAPTURE_MODE_RELAXED) == 0
+    try:
+        call()
+    finally:
+        rc = rt.hipStreamEndCapture(stream, ctypes.byref(graph))
+    assert rc == 0 and graph.value and hip.memory_stats()[0] == held
+    try:
+        assert rt.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0) == 0
+        for k in range(3):
+            r = np.random.default_rng(k)
+            for d, v in ((x, r.standard_normal((rows, H))), (g, r.standard_normal((rows, H))),
+                         (mean, 0.1 * r.standard_normal(rows)), (rstd, r.uniform(0.5, 2, rows))):
+                v = v.astype(np.float32)
+                hip.check(hip.lib.oxi_hip_memcpy_h2d(d.ptr, v.ctypes.data, v.nbytes))
+            call()
+            want = [o.numpy().copy() for o in (dx, dw, db)]
+            for o in (dx, dw, db):
+                hip.call("oxi_fill", o.ptr, o.size, -1.0)
+            hip.sync()
+            assert rt.hipGraphLaunch(exe, stream) == 0
+            hip.sync()
+            for o, v in zip((dx, dw, db), want):
+                np.testing.assert_array_equal(o.numpy().view(np.uint32), v.view(np.uint32))
+    finally:
+        if exe.value:
+            rt.hipGraphExecDestroy(exe)
+        rt.hipGraphDestroy(graph)
