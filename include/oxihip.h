@@ -361,8 +361,9 @@ int oxi_index_select_bwd(const float* g, int64_t outer, int64_t len, int64_t inn
  * soon as they are known (at forward time): up to 32768 of them in order on the
  * library stream, more on the library's second stream, after everything already
  * queued on the library stream; _apply makes the library stream wait for such a
- * plan and runs the segment sums of g for any (outer, inner) of the same ids. A plan may be applied more than once.
- * _plan_free releases it (after the library stream has passed its sort).
+ * plan and runs the segment sums of g for any (outer, inner) of the same ids.
+ * A plan may be applied more than once. _plan_free releases it (after the
+ * library stream has passed its sort).
  * Together they compute exactly what oxi_index_select_bwd computes. The
  * plan/apply split has no counterpart in the reference (its VJP is one call,
  * scatter_index_select, crates/oxi-autograd/src/ops.rs:741-769). */

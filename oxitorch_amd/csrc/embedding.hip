@@ -3,7 +3,7 @@
 // crates/oxi-tensor/src/lib.rs:665-703; scatter_index_select:
 // crates/oxi-autograd/src/ops.rs:741-769).
 //
-// Gather: out[o, k, :] = src[o, idx[k], :]. Each block copies GRPB (2) rows
+// Gather: out[o, k, :] = src[o, idx[k], :]. Each block copies GRPB (4) rows
 // with float4 accesses, the rows' loads issued together; threads per block
 // are the row's float4 count rounded up to whole waves.
 //
@@ -924,11 +924,16 @@ struct SortPlan {
 };
 
 // Ids up to which a plan is sorted on the library stream instead of the side
-// stream: ordering the two costs about 30 us and 35 us of host time, the sort
-// of 16384 ids 14. Plan, gather and VJP into (50257, 768), with nothing and with
-// three layer norms of the gathered rows between: 16384 ids 84 -> 69 and 126 ->
-// 129 us (the embedding-to-softmax chain of 16 x 1024 tokens 231 us either way), 32768 107 -> 97
-// and 202 -> 203, 64 64 -> 30 and 72 -> 41; 65536 ids 152 -> 141 but 342 -> 355.
+// stream: ordering the two costs about 20 us of a pass, the sort of 16384 ids
+// 14. A pass of plan, gather, k layer norms of the gathered rows, k of their
+// VJPs and the VJP into (50257, 768), from the side to the library stream, us:
+//   ids     k = 0         1              2              4              24
+//   64      51 -> 30      58 -> 39
+//   8192    68 -> 52      82.3 -> 81.6   112 -> 110     173 -> 166     753 -> 706
+//   16384   81 -> 70      106.4 -> 109.6 158.3 -> 159.4 264 -> 261     1321 -> 1271
+//   32768   116 -> 109    168.1 -> 171.8 257.7 -> 258.6 441 -> 436     2256 -> 2213
+// So a sort that one norm hides loses up to 3% in order, and passes with less
+// or more work between gain; with 65536 ids three norms lose (342 -> 355).
 constexpr int64_t PLAN_INLINE_MAX = 32768;
 
 int build_plan(const int64_t* idx, int64_t n, int64_t len, hipStream_t s, SortPlan* p) {

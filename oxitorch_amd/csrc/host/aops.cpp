@@ -276,8 +276,8 @@ Var narrow(const Var& x, int64_t dim, int64_t lo, int64_t hi, int64_t by) {
 // ---- index_select (ops.rs:498-517, 741-769) -----------------------------------------
 
 // The VJP's id sort is queued at forward time (oxi_index_select_bwd_plan):
-// few ids in order, many on the library's second stream, where it overlaps the
-// rest of the forward; the backward only waits for it and runs the segment sums.
+// up to 32768 ids in order, more on the library's second stream, where the sort
+// overlaps the forward; the backward only waits for it and runs the segment sums.
 Var index_select(const Var& x, int64_t dim, const std::vector<int64_t>& indices) {
   if (!is_grad_enabled() || !x.requires_grad()) return Var::leaf(t_index_select(x.value(), dim, indices), false);
   if (x.value().ndim() == 0) err_invalid("dim " + std::to_string(dim) + " out of range for 0-D tensor");
@@ -285,7 +285,7 @@ Var index_select(const Var& x, int64_t dim, const std::vector<int64_t>& indices)
   const Shape xs = x.value().shape;
   auto ids = device_i64(resolve_indices(indices, xs[d], d));
   const int64_t n = (int64_t)indices.size();
-  // the sort is queued first so that it overlaps the gather itself
+  // queued before the gather: a sort on the second stream overlaps it too
   void* raw = nullptr;
   hip_check(oxi_index_select_bwd_plan(static_cast<const int64_t*>(ids->ptr), n, xs[d], &raw));
   std::shared_ptr<void> plan(raw, [ids](void* p) { (void)oxi_index_select_bwd_plan_free(p); });

@@ -769,7 +769,7 @@ void launch_bwd_cfg(int cfg, bool odd, hipStream_t s, int64_t nblk, int nt, cons
         switch (cfg) {
           OXI_BWD(1024, 4)
           default:
-        norm_bwd_loop_k<MODE, LN><<<dim3((unsigned)nblk), dim3(BS), 0, s>>>(x, w, mean, rstd, g, dx, part, rows, h);
+            norm_bwd_loop_k<MODE, LN><<<dim3((unsigned)nblk), dim3(BS), 0, s>>>(x, w, mean, rstd, g, dx, part, rows, h);
         }
       }
   }
@@ -813,7 +813,8 @@ int launch_bwd(const float* x, const float* w, const float* b, const float* mean
   if (!need_part && nblk > (int64_t)cu_count() * 16) nblk = (int64_t)cu_count() * 16;
   if (nblk < 1) nblk = 1;
   // few rows, one to a group: blocks past the row blocks sum the columns
-  const bool few = need_part && !lsum && !is_softmax_act(ACT) && cfg && rows <= (ACT != ACT_NONE && tpr == 256 ? FEW_MAX_ACT256 : FEW_MAX) && rows <= nblk * gpb &&
+  const int few_max = ACT != ACT_NONE && tpr == 256 ? FEW_MAX_ACT256 : FEW_MAX;
+  const bool few = need_part && !lsum && !is_softmax_act(ACT) && cfg && rows <= few_max && rows <= nblk * gpb &&
                    nt_stores(rows * H * 4);
   const int64_t few_blocks = few ? ceil_div(H, 64) : 0;
   if (few) need_part = false;

@@ -32,17 +32,18 @@ constexpr int64_t WAVE_MAX_LEN = 2048;
 constexpr int64_t WAVE_SHORT_LEN = 128;
 // From SPLIT_MIN_LEN on, and with fewer strips than CUs, the strips are cut
 // into parts of a multiple of SPLIT_MIN_PART floats (four float4s a thread),
-// about SPLIT_BLOCKS_PER_CU a CU in all: the norm of 12.6M values 46000 ->
-// 12.9 us (3.9 TB/s), 1M values 1560 -> 7.1 us. The second launch costs about
-// 3 us, what one block takes for 30000 floats more.
+// about SPLIT_BLOCKS_PER_CU a CU in all: the norm of 12.6M values 46
+// ms -> 14 us of kernels (3.6 TB/s) with the input in the Infinity Cache (72
+// ms before from HBM), 1M values 1510 -> 10 us a call. The second launch takes
+// about 5 us, what one block takes for 50000 floats more.
 constexpr int64_t SPLIT_MIN_LEN = 65536;
 constexpr int64_t SPLIT_BLOCKS_PER_CU = 4;
 constexpr int64_t SPLIT_MIN_PART = 4096;
 constexpr int64_t SPLIT_MAX_PARTS = 1024;  // in a strip (LDS holds their states in a captured launch)
 // Strided strips of COLS_MIN_LEN positions or more, of up to COLS_MAX_OUT
-// outputs, go through LDS: the column sums of (16384, 768) 758 -> 59 us, of
+// outputs, go through LDS: the column sums of (16384, 768) 760-1200 -> 59 us, of
 // (1024, 16384) 68 -> 25 us, of (4096, 8000) 298 -> 42 us, the maxima of
-// (16384, 768) 760 -> 38 us. With more outputs a thread per output fills the
+// (16384, 768) 760-1200 -> 38 us. With more outputs a thread per output fills the
 // chip: (512, 65536) 42 us there against 57 us through LDS. Two and four
 // stages of loads in flight instead of one: 61-90 us at (16384, 768), the
 // staging then holding up the fold.

@@ -1,9 +1,10 @@
 // Register-resident row tiles for the row-wise kernels (norms, softmax).
 //
-// A row of H floats (H % 4 == 0, 16-byte aligned rows) is spread over a row
-// group of TPR threads: thread t holds float4 number k*TPR + t for k < NV, so
-// each load instruction of the group reads TPR*16 consecutive bytes (fully
-// coalesced). Out-of-range float4s are zero-filled and never stored.
+// A row of H floats is spread over a row group of TPR threads: thread t holds
+// float4 number k*TPR + t for k < NV, so each load instruction of the group
+// reads TPR*16 consecutive bytes (fully coalesced). Out-of-range float4s are
+// zero-filled and never stored. Rows lie at 16-byte addresses with H % 4 == 0,
+// or (the norms' ROW_ODD) anywhere, their last float4 overlapping the one before.
 // Rows are streamed (see ld_stream / st_stream below).
 #pragma once
 
