@@ -73,12 +73,14 @@ constexpr int bwd_waves_per_eu() { return LSUM && is_softmax_act(ACT) ? 4 : 1; }
 // float32 (a block's combine), those by slices in float64 (col_finish_k).
 // Layer norm's VJP of (64, 768) takes 4.8 us against 6.8 in two launches, of
 // (256, 4096) 5.9 against 12.1, with a folded tanh GELU 4.9 against 8.3 and 9.6
-// against 12.8; at 512 rows of 768 7.3 against 8.1 but 11.4 against 8.8 with the
-// GELU, at 1024 11.9 against 7.9. Rows of 256 threads have 4 waves a block to
+// against 12.8 (rows of 2049 to 4095 floats with the GELU up to 128 rows: (128,
+// 2552) 6.9 against 9.0, (160, 2552) 10.7 against 9.7); at 512 rows of 768 7.3
+// against 8.1 but 11.4 against 8.8 with the GELU, at 1024 11.9 against 7.9. Rows of 256 threads have 4 waves a block to
 // form a folded activation again: (32, 2048) 8.2 us either way, (64, 2048) 8.2
 // against 6.9.
 constexpr int FEW_MAX = 256;
 constexpr int FEW_MAX_ACT256 = 16;
+constexpr int FEW_MAX_TANH = 128;
 
 template <int GPB, bool LN, int ACT>
 __device__ __forceinline__ void few_columns(int cb, const float* __restrict__ x, const float* __restrict__ w,
@@ -813,7 +815,9 @@ int launch_bwd(const float* x, const float* w, const float* b, const float* mean
   if (!need_part && nblk > (int64_t)cu_count() * 16) nblk = (int64_t)cu_count() * 16;
   if (nblk < 1) nblk = 1;
   // few rows, one to a group: blocks past the row blocks sum the columns
-  const int few_max = ACT != ACT_NONE && tpr == 256 ? FEW_MAX_ACT256 : FEW_MAX;
+  const int few_max = ACT != ACT_NONE && tpr == 256                         ? FEW_MAX_ACT256
+                      : ACT == OXI_ACT_GELU_TANH && H > 2048 && H < 4096 ? FEW_MAX_TANH
+                                                                         : FEW_MAX;
   const bool few = need_part && !lsum && !is_softmax_act(ACT) && cfg && rows <= few_max && rows <= nblk * gpb &&
                    nt_stores(rows * H * 4);
   const int64_t few_blocks = few ? ceil_div(H, 64) : 0;

@@ -47,6 +47,12 @@ def test_same_bits_as_with_more_rows(hip, rows, H, act, layer, mode):
         np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("rows,H", [(128, 2552), (129, 2552), (129, 4096), (256, 4092)])
+def test_tanh_gelu_rows_of_a_few_thousand(hip, rows, H):
+    """Both sides of the rows where the folded tanh GELU goes back to two launches."""
+    test_same_bits_as_with_more_rows(hip, rows, H, "gelu_tanh", True, "ref")
+
+
 def test_only_one_of_dw_and_db(hip):
     print("norm few rows, one gradient", flush=True)
     r = np.random.default_rng(1)
