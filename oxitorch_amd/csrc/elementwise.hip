@@ -14,13 +14,15 @@
 //           tile and each lane a 4x4 block, read as float4 rows along the
 //           input's unit-stride dim and written as float4 columns along the
 //           output's innermost dim, so both coalesce with no LDS; dims of
-//           fewer than 4 take 64x64 tiles through LDS;
+//           fewer than 4, and long operations on tiny odd ones
+//           (map_through_lds), take 64x64 tiles through LDS;
 //   generic anything else: per-element index arithmetic.
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
 
 #include "internal.h"
+#include "map_route.h"
 #include "ops.h"
 #include "rowtile.h"
 
@@ -44,6 +46,14 @@ __device__ __forceinline__ float apply(const F& f, const float* v) {
   if constexpr (N == 1) return f(v[0]);
   else return f(v[0], v[1]);
 }
+
+// The fused activations and their VJPs are long.
+template <class F>
+constexpr OpLength op_length = OP_LONG;
+template <int OP>
+constexpr OpLength op_length<Unary<OP>> = unary_length(OP);
+template <int OP>
+constexpr OpLength op_length<Binary<OP>> = binary_length(OP);
 
 // ---------------------------------------------------------------------------
 // flat: y[i] = f(x0[i or 0], x1[i or 0]) for i < n.
@@ -511,6 +521,7 @@ int launch_map(F f, const char* what, float* y, const int64_t* ys, const float* 
         bool reg = p.shape[d] >= 4 && p.shape[jd] >= 4;
         for (int q = 0; q < p.ndim; ++q)
           if (p.shape[q] >= ((int64_t)1 << 31)) reg = false;
+        if (!vec && map_through_lds(op_length<F>, p.shape[jd], p.shape[d], blocks, cu_count())) reg = false;
         const int64_t rtiles = ceil_div(p.shape[d], RT) * ceil_div(p.shape[jd], RT) * batch;
         if (reg && rtiles < ((int64_t)1 << 31)) {
           const unsigned ntd = (unsigned)ceil_div(p.shape[d], RT), ntj = (unsigned)ceil_div(p.shape[jd], RT);

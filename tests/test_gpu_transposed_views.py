@@ -44,3 +44,23 @@ def test_bit_exact(hip, B, J, D, skip):
     run(lambda o: hip.call("oxi_binary", add, up, rm, tp, tv, o, rm, shape, 3), u + want_t, "u + t")
     run(lambda o: hip.call("oxi_binary", add, tp, tv, tp, tv, o, rm, shape, 3), want_t + want_t, "t + t")
     run(lambda o: hip.call("oxi_binary", add, tp, tv, cp, cv, o, rm, shape, 3), want_t + col, "t + column")
+
+
+@pytest.mark.parametrize("B,J,D", [(3, 4, 5), (100, 7, 7), (1030, 7, 7), (2, 11, 11), (130, 11, 9), (40, 11, 4), (2, 5, 1001),
+                                   (2100, 9, 5)])
+def test_long_operations(hip, B, J, D):
+    """Both sides of the sizes where long operations leave the registers for
+    LDS tiles: the bits of the same call on a contiguous copy."""
+    print("transposed, long", B, J, D, flush=True)
+    r = np.random.default_rng(B * J * D)
+    t, u = (r.uniform(0.1, 3, s).astype(np.float32) for s in ((B, D, J), (B, J, D)))
+    flat = hip.DeviceArray.from_numpy(np.ascontiguousarray(t.transpose(0, 2, 1)))
+    td, ud, shape, tv = hip.DeviceArray.from_numpy(t), hip.DeviceArray.from_numpy(u), (B, J, D), (D * J, 1, J)
+    rm = hip.row_major_strides(shape)
+    for what, got, want in (
+            ("tanh", hip.unary("tanh", td, x_strides=tv, shape=shape), hip.unary("tanh", flat)),
+            ("silu", hip.silu_fwd(td, x_strides=tv, shape=shape), hip.silu_fwd(flat)),
+            ("silu vjp", hip.silu_bwd(td, ud, x_strides=tv, g_strides=rm, shape=shape), hip.silu_bwd(flat, ud)),
+            ("gelu vjp", hip.gelu_bwd(td, ud, "tanh", x_strides=tv, g_strides=rm, shape=shape), hip.gelu_bwd(flat, ud, "tanh")),
+            ("pow", hip.binary("pow", td, ud, tv, rm, shape), hip.binary("pow", flat, ud, rm, rm, shape))):
+        np.testing.assert_array_equal(got.numpy().view(np.uint32), want.numpy().view(np.uint32), err_msg=what)

@@ -1,5 +1,6 @@
-"""Host side of the row-wise launches, no GPU: no grid passes the 2^32 threads
-that a launch can count (the rules, compiled here for the CPU)."""
+"""Host side of the launches, no GPU (the rules, compiled here for the CPU): no
+grid of the row-wise kernels passes the 2^32 threads that a launch can count,
+and which tiles transposed elementwise calls take."""
 
 import ctypes
 import subprocess
@@ -10,10 +11,15 @@ import pytest
 ROOT = Path(__file__).resolve().parents[1]
 
 SRC = r"""
+#include "map_route.h"
 #include "row_cfg.h"
 #include "softmax_mid.h"
 extern "C" int norm_fwd_cfg(int64_t rows, int64_t H) { return oxi::norm_fwd_cfg(rows, H); }
 extern "C" int block_threads(int tpr) { return oxi::row_block_threads(tpr); }
+extern "C" int through_lds(int unary, int op, int64_t J, int64_t D, int64_t blocks, int cus) {
+  return oxi::map_through_lds(unary < 0 ? oxi::OP_LONG : unary ? oxi::unary_length(op) : oxi::binary_length(op), J, D,
+                              blocks, cus);
+}
 extern "C" int64_t mid_outer_max(int64_t len, int64_t inner) { return oxi::mid_outer_max(len, inner); }
 extern "C" void mid_shape(int64_t outer, int64_t len, int64_t inner, int64_t* v) {
   const oxi::MidShape m = oxi::mid_shape(outer, len, inner);
@@ -72,3 +78,21 @@ def test_middle_dim_softmax_kernels(lib):
     for inner, few, most in ((2, 4, 16), (3, 4, 16), (4, 2, 8), (5, 2, 8), (1000, 2, 8)):
         got = {(m["nv"], m["nt"]) for m in (mid_shape(lib, 1, n, inner) for n in [*range(1, 5000), 10 ** 5, 10 ** 9])}
         assert got == {(0, 1024), (few, 256), (most, 256), (most, 1024)}
+
+
+def test_transposed_tiles(lib):
+    """Long operations on tiny odd extents go through LDS while few; short ones never."""
+    UN = ["neg", "abs", "sqrt", "rsqrt", "exp", "log", "log2", "log10", "sin", "cos", "tanh", "relu", "sigmoid"]
+
+    def lds(op, B, J, D):
+        kind, code = {"act": (-1, 0), "add": (0, 0), "pow": (0, 4)}.get(op) or (1, UN.index(op))
+        blocks = B * -(-J // 64) * -(-D // 64)
+        return bool(lib.through_lds(kind, code, *(ctypes.c_int64(v) for v in (J, D, blocks)), 256))
+
+    for op in ("act", "tanh", "sin", "sigmoid", "pow"):
+        assert all(lds(op, B, J, D) for B in (1, 25, 100, 1000) for J, D in ((4, 5), (7, 7), (11, 4), (4, 11))), op
+        assert not any(lds(op, B, J, D) for B in (1, 100) for J, D in ((31, 33), (33, 5), (1001, 5), (50, 63))), op
+        assert not lds(op, 100_000, 7, 7) and not lds(op, 5000, 11, 11), op
+    assert lds("act", 100, 11, 11) and not lds("act", 1000, 11, 11) and not lds("act", 1, 5, 1001)
+    assert lds("pow", 100, 5, 1001) and not lds("pow", 1000, 5, 1001) and lds("pow", 10_000, 4, 11)
+    assert not any(lds(op, B, 7, 7) for op in ("add", "neg", "abs", "relu") for B in (1, 100, 10_000))
