@@ -525,11 +525,16 @@ void norm_bwd_k(const float* __restrict__ x, const float* __restrict__ w,
         }
       }
     }
-  } else if (TPR * NV > 2048 || (int64_t)rows <= ngroups) {
-    // at most one row per group (e.g. 4096 rows of 768): nothing to prefetch;
+  } else if constexpr (TPR * NV > 2048) {
     // rows of 1024 threads: no registers for a second row (128 VGPRs a lane)
 #pragma unroll 1
     for (; row < rows; row += ngroups) {
+      fetch(xa, ga, ia, ma, row);
+      process(xa, ga, ia, ma, row);
+    }
+  } else if ((int64_t)rows <= ngroups) {
+    // at most one row per group (e.g. 4096 rows of 768): nothing to prefetch
+    if (row < rows) {
       fetch(xa, ga, ia, ma, row);
       process(xa, ga, ia, ma, row);
     }

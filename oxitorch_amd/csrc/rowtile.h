@@ -121,8 +121,10 @@ inline bool nt_stores(int64_t bytes) { return bytes < (int64_t)OXI_NT_STORE_LO |
 // before (both lanes form and write the same values) and are left out of sums.
 enum RowKind { ROW_VEC = 0, ROW_FULL = 1, ROW_ODD = 2 };
 
+// constexpr: for ROW_FULL the count is then a constant before inlining, as the
+// kernels' unrolling and registers need it (512 threads x 4: 163 VGPRs, 175 without).
 template <int KIND>
-__device__ __forceinline__ int row_slots(int H) { return KIND == ROW_ODD ? (H + 3) >> 2 : H >> 2; }
+__device__ __forceinline__ constexpr int row_slots(int H) { return KIND == ROW_ODD ? (H + 3) >> 2 : H >> 2; }
 
 // Slot c of an odd row (slots past the last re-read it).
 __device__ __forceinline__ f4 ld_odd(const float* __restrict__ row, int H, int c) {
