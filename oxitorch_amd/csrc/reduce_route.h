@@ -44,7 +44,7 @@ constexpr int64_t SPLIT_MAX_PARTS = 1024;  // in a strip (LDS holds their states
 // outputs, go through LDS: the column sums of (16384, 768) 760-1200 -> 59 us, of
 // (1024, 16384) 68 -> 25 us, of (4096, 8000) 298 -> 42 us, the maxima of
 // (16384, 768) 760-1200 -> 38 us. With more outputs a thread per output fills the
-// chip: (512, 65536) 42 us there against 57 us through LDS. Two and four
+// chip: (512, 65536) 22 us there against 57 through LDS. Two and four
 // stages of loads in flight instead of one: 61-90 us at (16384, 768), the
 // staging then holding up the fold.
 constexpr int64_t COLS_MIN_LEN = 64;
@@ -65,6 +65,13 @@ constexpr int COLS_THREADS = 512 + 64;  // its loading threads and the wave that
 constexpr int64_t COLS_ROUND_LEN = 128;
 constexpr int64_t COLS_ROUND_LEN_NARROW = 64;
 constexpr int64_t COLS_MAX_ROUNDS = 8;
+
+// Other strided strips take a thread per output, its 16 loads in flight, or from
+// VEC_MIN_OUT outputs a CU on, where a quarter of the threads still fill the
+// chip, a thread per four, 8 float4s in flight: sums of (29, 75576) 5.2 us
+// against 7.2, of (1000, 20480) 29.5 against 73.5, of (128, 327680) 25 against
+// 29, but of (16, 655360) 8.5 against 7.4, of (4, 16777216) 92 against 55.
+constexpr int64_t VEC_MIN_OUT = 2048;
 
 constexpr bool is_arg(int k) { return k == OXI_REDUCE_ARGMAX || k == OXI_REDUCE_ARGMIN; }
 // kinds whose result depends on the order of the fold
@@ -138,12 +145,9 @@ inline ReduceRoute reduce_route(int kind, const RPlan& p, int64_t nout, const fl
       r.threads = COLS_THREADS;
       return r;
     }
-    // a thread per output, 16 loads in flight, where the float4 kernel keeps a
-    // quarter of the threads busy: the sums over dim 1 of (16384 / 4, 100, 4)
-    // 5.0 us against 41, of (256, 64, 64) 4.6 against 5.1
-    r.vec = false;
   }
-  r.kernel = !is_arg(kind) && r.vec && aligned(out) ? ReduceKernel::Vec : ReduceKernel::Threads;
+  r.kernel = !is_arg(kind) && r.vec && aligned(out) && nout >= VEC_MIN_OUT * (int64_t)cus ? ReduceKernel::Vec
+                                                                                         : ReduceKernel::Threads;
   r.blocks = std::min(ceil(r.kernel == ReduceKernel::Vec ? nout / 4 : nout, 256), (int64_t)cus * 64);
   return r;
 }

@@ -92,6 +92,12 @@ def test_narrow_rows_of_outputs(hip, shape, full, dim):
                                       ref.reduce(kind, np.ascontiguousarray(x), dim), err_msg=kind)
 
 
+@pytest.mark.parametrize("shape", [(17, 524288), (17, 524284), (9, 1024, 1, 512), (8, 524290)])
+def test_one_or_four_outputs_a_thread(hip, shape):
+    print("reduce many outputs", shape, flush=True)
+    test_narrow_rows_of_outputs(hip, shape, shape, 0)
+
+
 @pytest.mark.parametrize("rows,cols,dim", [(4, 70000, 1), (4, 700, 1), (700, 20, 0)])
 def test_first_winner_and_nan_rules(hip, rows, cols, dim):
     """Ties go to the first position, a NaN counts only at position 0, strips

@@ -147,6 +147,18 @@ def test_grids_stay_below_the_thread_limit(lib, length):
             assert r["kernel"] == "threads"
 
 
+@pytest.mark.parametrize("kind", KINDS)
+def test_four_outputs_a_thread(lib, kind):
+    """From 2048 outputs a CU on, with aligned rows of a multiple of 4; not for argmax and argmin."""
+    arg = kind in ("argmax", "argmin")
+    for length in (2, 29, 1000):
+        for shape, dim in (((length, 2048 * CUS), 0), ((length, 512, 4 * CUS), 0), ((2048 * CUS // 64, length, 64), 1)):
+            assert route(lib, shape, dim, kind)["kernel"] == ("threads" if arg else "vec"), shape
+            assert route(lib, shape, dim, kind, x=4)["kernel"] == "threads"
+    for shape in ((29, 2048 * CUS - 4), (29, 2048 * CUS + 2), (29, 12596, 1, 6), (1000, 20000)):
+        assert route(lib, shape, 0, kind)["kernel"] == "threads", shape
+
+
 def test_parts_of_a_strip(lib):
     """They cover it, none empty, and their states fit a block's LDS."""
     for n, length in itertools.product((1, 2, 3, 17, 255), (65536, 65537, 1048583, 10 ** 8, 2 ** 31)):
